@@ -29,8 +29,10 @@
 //            visible pair), then dQ = dS K * scale from the stored tiles --
 //            no second S and dP, at the price of the dS traffic.
 //
-// fp32 inputs (and head_dim outside the MFMA set, up to 1024) run on a SIMT
-// path: one wavefront per row, exact fp32 arithmetic.
+// fp32 inputs with head_dim 64 or 128 and 16-byte aligned rows run the fp32
+// matrix kernels of attention_f32.h; the other fp32 calls (and 16-bit ones
+// with head_dim outside the MFMA set, up to 1024) a SIMT path: one wavefront
+// per row, exact fp32 arithmetic.
 //
 // Workgroup order is XCD-aware: the 8 XCDs receive workgroups round-robin, so
 // block ids are remapped to give every XCD a contiguous range of
@@ -2786,6 +2788,8 @@ attn_bwd_dkdv_simt(BwdArgs a, int D) {
   }
 }
 
+#include "attention_f32.h"
+
 // ------------------------------------------------------------- host side --
 bool mfma_head_dim(int64_t d) { return d == 16 || d == 32 || d == 64 || d == 128 || d == 256; }
 
@@ -2987,9 +2991,10 @@ int bwd_impl(const BwdArgs& a, int64_t D, bool mfma, hipStream_t st) {
   return check_launch("attention backward (dk/dv, simt)");
 }
 
-// Row strides must keep 16-byte alignment of every row for the MFMA path.
-bool rows_aligned(const void* p, int64_t sb, int64_t sh, int64_t ss) {
-  return aligned16(p) && sb % 8 == 0 && sh % 8 == 0 && ss % 8 == 0;
+// Row strides must keep 16-byte alignment of every row for the MFMA paths.
+bool rows_aligned(const void* p, int64_t sb, int64_t sh, int64_t ss, int dtype) {
+  const int64_t vec = 16 / dtype_size(dtype);
+  return aligned16(p) && sb % vec == 0 && sh % vec == 0 && ss % vec == 0;
 }
 
 int check_dims(int64_t B, int64_t H, int64_t Hkv, int64_t Tq, int64_t Tkv, int64_t D) {
@@ -3032,17 +3037,23 @@ int attention_fwd(const void* q, const void* k, const void* v, void* o, float* l
   a.scale = (float)(1.0 / sqrt((double)D));
   a.rope = rope;
   hipStream_t st = (hipStream_t)stream;
-  const bool mfma = dtype != kF32 && mfma_head_dim(D) &&
-                    rows_aligned(q, a.sq_b, a.sq_h, a.sq_s) &&
-                    rows_aligned(k, a.sk_b, a.sk_h, a.sk_s) &&
-                    rows_aligned(v, a.sv_b, a.sv_h, a.sv_s) && aligned16(o) &&
-                    a.so_s % 4 == 0 && a.so_b % 4 == 0 && a.so_h % 4 == 0;
+  const bool aligned = rows_aligned(q, a.sq_b, a.sq_h, a.sq_s, dtype) &&
+                       rows_aligned(k, a.sk_b, a.sk_h, a.sk_s, dtype) &&
+                       rows_aligned(v, a.sv_b, a.sv_h, a.sv_s, dtype) && aligned16(o) &&
+                       a.so_s % 4 == 0 && a.so_b % 4 == 0 && a.so_h % 4 == 0;
+  const bool mfma = dtype != kF32 && mfma_head_dim(D) && aligned;
   if (rope.cos != nullptr && !(mfma && (D == 64 || D == 128)))
     return fail(TRI_EINVAL, "attention with rope: needs 16-bit q/k/v with head_dim 64 or 128 and "
                 "16-byte aligned rows (dtype %d, head_dim %lld)", dtype, (long long)D);
   if (mfma) {
     if (dtype == kBF16) return fwd_mfma<bf16_t>(a, D, st);
     return fwd_mfma<f16_t>(a, D, st);
+  }
+  // 33 times the SIMT path's speed at [4, 12, 1024, 64]; head_dims 16 and 32
+  // fill only part of the tile layout's rows and stay on that path
+  if (dtype == kF32 && aligned) {
+    if (D == 64) return fwd_f32<64>(a, st);
+    if (D == 128) return fwd_f32<128>(a, st);
   }
   TRI_DISPATCH_FLOAT(dtype, T, return fwd_simt<T>(a, D, st));
   return TRI_OK;
@@ -3089,12 +3100,12 @@ int attention_bwd(const void* dout, const void* q, const void* k, const void* v,
       if (s[i] % 4 != 0) return false;
     return aligned16(dq) && aligned16(dk) && aligned16(dv);
   }();
-  const bool mfma = dtype != kF32 && mfma_head_dim(D) &&
-                    rows_aligned(q, a.sq_b, a.sq_h, a.sq_s) &&
-                    rows_aligned(k, a.sk_b, a.sk_h, a.sk_s) &&
-                    rows_aligned(v, a.sv_b, a.sv_h, a.sv_s) &&
-                    rows_aligned(dout, a.sdo_b, a.sdo_h, a.sdo_s) &&
-                    rows_aligned(o, a.so_b, a.so_h, a.so_s) && out_ok;
+  const bool aligned = rows_aligned(q, a.sq_b, a.sq_h, a.sq_s, dtype) &&
+                       rows_aligned(k, a.sk_b, a.sk_h, a.sk_s, dtype) &&
+                       rows_aligned(v, a.sv_b, a.sv_h, a.sv_s, dtype) &&
+                       rows_aligned(dout, a.sdo_b, a.sdo_h, a.sdo_s, dtype) &&
+                       rows_aligned(o, a.so_b, a.so_h, a.so_s, dtype) && out_ok;
+  const bool mfma = dtype != kF32 && mfma_head_dim(D) && aligned;
   hipStream_t st = (hipStream_t)stream;
   if (rope.cos != nullptr) {
     if (!(mfma && (D == 64 || D == 128)))
@@ -3113,6 +3124,10 @@ int attention_bwd(const void* dout, const void* q, const void* k, const void* v,
       a.ds = ds_ws;
       a.ds_bh = (int64_t)(need / 2 / (size_t)(B * H));
     }
+  }
+  if (dtype == kF32 && aligned) {
+    if (D == 64) return bwd_f32<64>(a, st);
+    if (D == 128) return bwd_f32<128>(a, st);
   }
   TRI_DISPATCH_FLOAT(dtype, T, return bwd_impl<T>(a, D, mfma, st));
   return TRI_OK;
@@ -3235,8 +3250,8 @@ int decode_launch(const void* q, const void* k, const void* v, void* o, float* l
   a.sk_b = strides[3]; a.sk_h = strides[4]; a.sk_s = strides[5];
   a.sv_b = strides[6]; a.sv_h = strides[7]; a.sv_s = strides[8];
   a.so_b = strides[9]; a.so_h = strides[10];
-  if (!aligned16(q) || a.sq_b % 8 || a.sq_h % 8 || !rows_aligned(k, a.sk_b, a.sk_h, a.sk_s) ||
-      !rows_aligned(v, a.sv_b, a.sv_h, a.sv_s))
+  if (!aligned16(q) || a.sq_b % 8 || a.sq_h % 8 || !rows_aligned(k, a.sk_b, a.sk_h, a.sk_s, dtype) ||
+      !rows_aligned(v, a.sv_b, a.sv_h, a.sv_s, dtype))
     return fail(TRI_EINVAL, "attention decode: q, k, v rows must be 16-byte aligned");
   a.B = (int)B; a.H = (int)H; a.Hkv = (int)Hkv; a.Tkv = (int)Tkv;
   a.n_splits = dec_splits(B, Hkv, Tkv);

@@ -285,3 +285,26 @@ def test_attention_pingpong_grid():
     _check_heads(torch.float16, 2, 256, 64, 731, 128, True, [(0, 0), (1, 63)], seed=22,
                  grads=True)
     _check_heads(torch.bfloat16, 2, 256, 256, 600, 128, False, [(0, 5), (1, 250)], seed=23)
+
+
+# fp32 at head_dim 64 and 128 runs the fp32 matrix kernels: 64-row tiles (128
+# query rows a workgroup in the head_dim 128 forward) swept in two 32-row
+# halves.  Edges: one row, rows and keys just over and under 32, 64 and 128,
+# a half without keys, Tq != Tkv under the top-left mask, GQA, strided module
+# views; the last, rows that are not 16-byte aligned, stays on the SIMT path.
+# Tolerance 1e-5: fp32 sums of at most 300 terms of order 1.
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize(("b", "h", "hkv", "tq", "tkv", "layout"), [
+    (1, 1, 1, 1, 1, "bhtd"), (1, 2, 2, 31, 33, "bhtd"), (2, 2, 1, 65, 63, "bthd"),
+    (1, 4, 2, 129, 127, "bthd"), (1, 2, 2, 1, 300, "bhtd"), (1, 2, 1, 300, 20, "bhtd"),
+    (4, 4, 2, 192, 192, "bthd"), (2, 8, 8, 257, 257, "bhtd")])
+def test_attention_fp32_matrix_kernels(b, h, hkv, tq, tkv, layout, causal, head_dim):
+    _check(torch.float32, b, h, hkv, tq, tkv, head_dim, causal, seed=61, layout=layout)
+
+
+def test_attention_fp32_unaligned_rows():
+    x = [randn((1, 2, 70, 67), torch.float32, 71 + i)[..., 1:65] for i in range(3)]
+    o = tritium.attention(*x)
+    eo, _ = oracle.attention.forward(*(np32(t) for t in x), True)
+    assert_close(o, eo, 1e-5, 1e-5)
