@@ -2397,7 +2397,7 @@ attn_bwd_dq_ds(BwdArgs a) {
 // shuffles, the wavefronts through LDS, and each workgroup writes its chunk's
 // unnormalised (m, l, o) per head to a workspace that attn_decode_combine
 // merges over the chunks (o = sum o_c 2^(m_c - M) / sum l_c 2^(m_c - M)).
-constexpr int kDecWaves = 4;
+constexpr int kDecWaves = 4;              // wavefronts of attn_decode_kernel
 constexpr int kDecMinChunk = 256;        // keys per chunk at least
 // workgroups to aim for: 512 against 2048 (graph replays, same box) took
 // [8, 32, 8, 8192, 128] 58.3 -> 53.6-54.4 us and [8, 32, 32, 4096, 128]
@@ -2451,19 +2451,52 @@ __device__ __forceinline__ void dec_merge(float& m, float& l, float (&o)[N], flo
   m = mx;
 }
 
-template <typename T, int D, int G>
-__global__ void __launch_bounds__(64 * kDecWaves)
-attn_decode_kernel(DecArgs a) {
+// LDS of a workgroup of `waves` wavefronts: per wavefront and head m, l, o[D].
+constexpr int dec_lds_floats(int waves, int heads, int D) { return waves * heads * (D + 2); }
+
+// Merge the wavefronts' states of every head (sm: [WAVES][G] m, then l, then
+// o[D]) and write the chunk's partials, or o and lse when one chunk holds the
+// whole cache (as the combine kernel would form them from that one partial,
+// its weight 2^(m - m) = 1, so no second launch).  Thread d owns dimension d.
+template <typename T, int D, int G, int WAVES>
+__device__ __forceinline__ void dec_write(const DecArgs& a, const float* sm, int b, int hk,
+                                          int group, int split) {
+  const float* sl = sm + WAVES * G;
+  const float* so = sl + WAVES * G;
+  for (int t = threadIdx.x; t < group * D; t += 64 * WAVES) {
+    const int g = t / D, d = t % D;
+    float mm = sm[g], ll = sl[g], oo[1] = {so[g * D + d]};
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) {
+      const float o2[1] = {so[(w * G + g) * D + d]};
+      dec_merge<1>(mm, ll, oo, sm[w * G + g], sl[w * G + g], o2);
+    }
+    const int hq = hk * group + g;
+    if (a.n_splits == 1) {
+      ((T*)a.o + b * a.so_b + hq * a.so_h)[d] = from_f32<T>(ll > 0.f ? oo[0] / ll : 0.f);
+      if (d == 0) a.lse[(int64_t)b * a.H + hq] = (mm + log2f(ll)) * kLn2;
+    } else {
+      float* dst = a.part + (((int64_t)b * a.H + hq) * a.n_splits + split) * (D + 2);
+      dst[2 + d] = oo[0];
+      if (d == 0) {
+        dst[0] = mm;
+        dst[1] = ll;
+      }
+    }
+  }
+}
+
+// One chunk of keys on the vector ALU: fp32 products and weights.  `sm` holds
+// dec_lds_floats(WAVES, G, D) floats.
+template <typename T, int D, int G, int WAVES>
+__device__ __forceinline__ void dec_chunk(const DecArgs& a, float* sm, int b, int hk, int group,
+                                          int split) {
   constexpr int LPK = D / 8;     // lanes per key row
   constexpr int KPW = 64 / LPK;  // keys per wavefront step
-  __shared__ float sm[kDecWaves][G], sl[kDecWaves][G], so[kDecWaves][G][D];
+  float* sl = sm + WAVES * G;
+  float* so = sl + WAVES * G;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int sub = lane / LPK, part = lane % LPK;
-  int bid = blockIdx.x;
-  const int split = bid % a.n_splits;
-  bid /= a.n_splits;
-  const int hk = bid % a.Hkv, b = bid / a.Hkv;
-  const int group = a.H / a.Hkv;
   const int kv0 = split * a.chunk;
   const int kv1 = min(a.Tkv, kv0 + a.chunk);
 
@@ -2489,7 +2522,7 @@ attn_decode_kernel(DecArgs a) {
   // kDecUnroll key rows per lane are loaded before any is used (memory-level
   // parallelism for a latency-bound stream); the LPK lanes of a key row share
   // its bounds, so the shuffles below only combine lanes active together
-  constexpr int kStride = kDecWaves * KPW;
+  constexpr int kStride = WAVES * KPW;
   for (int kv = kv0 + wave * KPW + sub; kv < kv1; kv += kDecUnroll * kStride) {
     u32x4 kr[kDecUnroll], vr[kDecUnroll];
 #pragma unroll
@@ -2542,41 +2575,232 @@ attn_decode_kernel(DecArgs a) {
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       if (part == 0) {
-        sm[wave][g] = m[g];
-        sl[wave][g] = l[g];
+        sm[wave * G + g] = m[g];
+        sl[wave * G + g] = l[g];
       }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) so[wave][g][part * 8 + i] = o[g][i];
+      for (int i = 0; i < 8; ++i) so[(wave * G + g) * D + part * 8 + i] = o[g][i];
     }
   }
   __syncthreads();
-  // merge the wavefronts; thread d < D owns dimension d of every head
-  for (int g = 0; g < group && g < G; ++g) {
-    if (threadIdx.x < D) {
-      float mm = sm[0][g], ll = sl[0][g], oo[1] = {so[0][g][threadIdx.x]};
+  dec_write<T, D, G, WAVES>(a, sm, b, hk, group, split);
+}
+
+template <typename T, int D, int G, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
+attn_decode_kernel(DecArgs a) {
+  __shared__ float sm[dec_lds_floats(WAVES, G, D)];
+  const int split = blockIdx.x % a.n_splits, bh = blockIdx.x / a.n_splits;
+  dec_chunk<T, D, G, WAVES>(a, sm, bh / a.Hkv, bh % a.Hkv, a.H / a.Hkv, split);
+}
+
+// The same chunk on the matrix cores.  With G query heads a key row costs the
+// kernel above about 16 + 24 G vector instructions per 8 elements, more than
+// the time to read it from HBM at G >= 4; here the heads are the 16 columns
+// of S^T = K Q^T and O^T = V^T P^T (v_mfma_f32_16x16x32), so a 32-key tile
+// costs one softmax of 8 registers whatever the group.  Every wavefront
+// streams its own 32-key tiles: K and V rows by DMA into a private LDS ring
+// (16 KB a wavefront: one tile at head_dim 128, two at 64; eight wavefronts a
+// CU overlap each other's loads and arithmetic better than four with twice
+// the ring, [8, 32, 8, 8192, 128] 46.4 against 48.4 us), no barrier until the
+// end.  Register r of S^T block u
+// holds key 16 u + 4 g + r (g = lane >> 4), which is the operand order of the
+// P^T that follows; V^T comes from transposing LDS reads of the same keys.
+// P enters the product as a sum of three 16-bit terms, which hold all 24 bits
+// of the fp32 weight.  (For fp16, whose terms would lose bits below 2^-24,
+// weights are formed 2^7 larger; the reference point of the partials accounts
+// for it.)  A non-finite key or value turns such a sum into NaN where the
+// plain product may be infinite, so a chunk that ends in any NaN is done
+// again by dec_chunk.
+//
+// Bound: HBM.  Graph replays, same box, dec_chunk's kernel -> this one:
+// [8, 32, 8, 8192, 128] 54.0 -> 47.0 us (5.7 TB/s with the combine), [32, 32,
+// 8, 2048, 128] 53.2 -> 47.8, [1, 32, 8, 4096, 128] 18.2 -> 11.6, [10, 12, 3,
+// 9149, 64] 25.1 -> 21.9, [3, 32, 4, 16000, 64] 33.0 -> 17.4, [1, 16, 2,
+// 2000, 64] 18.9 -> 7.5; with groups of one and two heads it is equal or up
+// to 4% slower, so those stay on the kernel above.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <typename T>
+__device__ __forceinline__ f32x4 mma16(typename Mfma<T>::V a, typename Mfma<T>::V b, f32x4 c) {
+  if constexpr (std::is_same<T, bf16_t>::value)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+// Max and sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48.
+__device__ __forceinline__ float quarter_max(float x) {
+  const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return xor32_max(fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])));
+}
+__device__ __forceinline__ float quarter_sum(float x) {
+  x += __shfl_xor(x, 16, kWave);
+  return x + __shfl_xor(x, 32, kWave);
+}
+
+constexpr int kDecMWaves = 4;
+constexpr int kDecRing = 16384;  // bytes per wavefront
+
+template <typename T, int D>
+__global__ void __launch_bounds__(64 * kDecMWaves, 2)
+attn_decode_mfma(DecArgs a) {
+  typedef typename Mfma<T>::V V;
+  typedef BTile<D> P;
+  constexpr int W = kDecMWaves, GMAX = 8, KS = D / 32, MT = D / 16;
+  constexpr int TILE = 32 * P::RB, RING = kDecRing, STAGES = RING / (2 * TILE);
+  constexpr int DMAS = TILE / 1024;          // per 32-row tile
+  constexpr int NV = D == 128 ? 4 : 2;       // DMAs after which the swizzle repeats
+  constexpr float SHIFT = std::is_same<T, f16_t>::value ? 7.f : 0.f;
+  static_assert(STAGES >= 1 && dec_lds_floats(W, GMAX, D) * 4 <= W * RING, "LDS");
+  __shared__ __attribute__((aligned(1024))) char smem[W * RING];
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int l16 = lane & 15, g = lane >> 4;
+  const int split = blockIdx.x % a.n_splits, bh = blockIdx.x / a.n_splits;
+  const int b = bh / a.Hkv, hk = bh % a.Hkv, group = a.H / a.Hkv;
+  const int kv0 = split * a.chunk, kv1 = min(a.Tkv, kv0 + a.chunk);
+  const T* kp = (const T*)a.k + b * a.sk_b + hk * a.sk_h;
+  const T* vp = (const T*)a.v + b * a.sv_b + hk * a.sv_h;
+  char* ring = smem + wave * RING;
+  // this wavefront's tiles: keys kv0 + 32 wave, + 32 W, ...
+  const int first = kv0 + 32 * wave;
+  const int n = first < kv1 ? (kv1 - first + 32 * W - 1) / (32 * W) : 0;
+
+  // byte offsets of this lane's 16 bytes within DMA i (i mod NV) from the
+  // DMA's first row; 32 bits hold them for rows up to 64 MB apart
+  const bool fast = a.sk_s < (1 << 25) && a.sv_s < (1 << 25) && a.sk_s >= 0 && a.sv_s >= 0;
+  uint32_t ko[NV], vo[NV];
 #pragma unroll
-      for (int w = 1; w < kDecWaves; ++w) {
-        const float o2[1] = {so[w][g][threadIdx.x]};
-        dec_merge<1>(mm, ll, oo, sm[w][g], sl[w][g], o2);
+  for (int i = 0; i < NV; ++i) {
+    const int r = lane / P::GR, c = (lane % P::GR) ^ P::key(i * P::DMA_ROWS + r);
+    ko[i] = (uint32_t)(r * (fast ? a.sk_s : 0) + c * 8) * sizeof(T);
+    vo[i] = (uint32_t)(r * (fast ? a.sv_s : 0) + c * 8) * sizeof(T);
+  }
+  auto issue = [&](int t) {
+    const int r0 = first + 32 * W * t;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_addr(ring + (t % STAGES) * 2 * TILE));
+    if (fast && r0 + 32 <= a.Tkv) {
+      const T* kt = kp + (int64_t)r0 * a.sk_s;
+      const T* vt = vp + (int64_t)r0 * a.sv_s;
+#pragma unroll
+      for (int i = 0; i < DMAS; ++i) {
+        dma16s_nt(kt + i * P::DMA_ROWS * a.sk_s, ko[i % NV], dst + i * 1024);
+        dma16s_nt(vt + i * P::DMA_ROWS * a.sv_s, vo[i % NV], dst + TILE + i * 1024);
       }
-      if (a.n_splits == 1) {
-        // one chunk holds the whole cache: o and lse directly, as the
-        // combine kernel would form them from this one partial (its weight
-        // 2^(m - m) = 1), so no second launch
-        const int hq = hk * group + g;
-        T* orow = (T*)a.o + b * a.so_b + hq * a.so_h;
-        orow[threadIdx.x] = from_f32<T>(ll > 0.f ? oo[0] / ll : 0.f);
-        if (threadIdx.x == 0) a.lse[(int64_t)b * a.H + hq] = (mm + log2f(ll)) * kLn2;
-      } else {
-        float* dst = a.part + (((int64_t)b * a.H + hk * group + g) * a.n_splits + split) * (D + 2);
-        dst[2 + threadIdx.x] = oo[0];
-        if (threadIdx.x == 0) {
-          dst[0] = mm;
-          dst[1] = ll;
-        }
+    } else {  // rows past the cache: the last one
+#pragma unroll
+      for (int i = 0; i < DMAS; ++i) {
+        const int trow = i * P::DMA_ROWS + lane / P::GR;
+        const int c = (lane % P::GR) ^ P::key(trow);
+        const int64_t row = min(r0 + trow, a.Tkv - 1);
+        dma16_nt(kp + row * a.sk_s + c * 8, dst + i * 1024);
+        dma16_nt(vp + row * a.sv_s + c * 8, dst + TILE + i * 1024);
       }
     }
+  };
+  V qf[KS];  // lane l16's head, elements 32 st + 8 g ..; zeros past the group
+#pragma unroll
+  for (int st = 0; st < KS; ++st)
+    qf[st] = l16 < group ? ld8((const T*)a.q + b * a.sq_b + (int64_t)(hk * group + l16) * a.sq_h +
+                               32 * st + 8 * g)
+                         : zero8<T>();
+  f32x4 o[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) o[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, nm = SHIFT, l = 0.f;
+#pragma unroll
+  for (int t = 0; t < STAGES; ++t)
+    if (t < n) issue(t);
+  for (int t = 0; t < n; ++t) {
+    // tile t has landed once only the younger tiles' DMAs are outstanding
+    if (t + STAGES <= n) wait_vmcnt<(STAGES - 1) * 2 * DMAS>();
+    else wait_vmcnt<0>();
+    asm volatile("" ::: "memory");
+    const char* Ks = ring + (t % STAGES) * 2 * TILE;
+    const char* Vs = Ks + TILE;
+    f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int st = 0; st < KS; ++st)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        s[u] = mma16<T>(*reinterpret_cast<const V*>(Ks + P::off(16 * u + l16, 4 * st + g)), qf[st], s[u]);
+    const int kb = first + 32 * W * t;
+    if (kb + 32 > kv1) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          s[u][r] = 16 * u + r > kv1 - 1 - kb - 4 * g ? -INFINITY : s[u][r];
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      mx = fmaxf(fmaxf(fmaxf(s[u][0], s[u][1]), fmaxf(s[u][2], s[u][3])), mx);
+    mx = quarter_max(mx) * a.sl2;
+    if (__builtin_amdgcn_ballot_w64(mx > m + 8.f) != 0) {  // lazy rescaling, as in attn_fwd_v2
+      const float m_new = fmaxf(m, mx);
+      const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);
+      m = m_new;
+      nm = m == -INFINITY ? SHIFT : SHIFT - m;
+      l *= alpha;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) o[mt] *= alpha;
+    }
+    V p[3];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float x = fast_exp2(fmaf(s[u][r], a.sl2, nm));
+        l += x;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          p[k][4 * u + r] = (T)x;
+          x -= (float)p[k][4 * u + r];
+        }
+      }
+    // V^T operands: in each 16-lane group, lane s addresses row 4 g + (s >> 2)
+    // at column 4 (s & 3) of the 16, and lane j receives column j's four rows
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      typedef short v4s __attribute__((ext_vector_type(4)));
+      typedef __attribute__((address_space(3))) v4s lds_v4s;
+      const int r0 = 4 * g + (l16 >> 2), c = 2 * mt + ((l16 & 3) >> 1), sub = (l16 & 1) * 8;
+      const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(lds_addr(Vs + P::off(r0, c) + sub)));
+      const v4s hi =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(lds_addr(Vs + P::off(16 + r0, c) + sub)));
+      const V v = __builtin_bit_cast(V, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+      for (int k = 0; k < 3; ++k) o[mt] = mma16<T>(v, p[k], o[mt]);
+    }
+    // every LDS read of this stage has returned before its DMA is reissued
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (t + STAGES < n) issue(t + STAGES);
   }
+  l = quarter_sum(l);
+
+  bool bad = l != l;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bad |= o[mt][r] != o[mt][r];
+  float* sm = reinterpret_cast<float*>(smem);
+  float* sl = sm + W * GMAX;
+  float* so = sl + W * GMAX;
+  if (__syncthreads_or(bad && l16 < group)) {
+    dec_chunk<T, D, GMAX, W>(a, sm, b, hk, group, split);
+    return;
+  }
+  if (l16 < group) {
+    if (g == 0) {
+      sm[wave * GMAX + l16] = m == -INFINITY ? m : m - SHIFT;
+      sl[wave * GMAX + l16] = l;
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      *reinterpret_cast<f32x4*>(so + (wave * GMAX + l16) * D + 16 * mt + 4 * g) = o[mt];
+  }
+  __syncthreads();
+  dec_write<T, D, GMAX, W>(a, sm, b, hk, group, split);
 }
 
 // o[b, h] and lse[b, h] from the chunks' (m, l, o): the chunk maxima and
@@ -3254,7 +3478,14 @@ int decode_launch(const void* q, const void* k, const void* v, void* o, float* l
       !rows_aligned(v, a.sv_b, a.sv_h, a.sv_s, dtype))
     return fail(TRI_EINVAL, "attention decode: q, k, v rows must be 16-byte aligned");
   a.B = (int)B; a.H = (int)H; a.Hkv = (int)Hkv; a.Tkv = (int)Tkv;
+  // A short cache with one or two heads per kv head: one workgroup of 16
+  // wavefronts per (batch, kv head) takes two passes of loads over its keys
+  // and writes the result, which costs less than the second launch it saves
+  // ([1, 12, 12, 517, 64] 7.3 -> 5.3 us of kernels, 17.0 -> 14.4 us a call;
+  // at twice the bytes, 1000 keys of 128, 11.7 -> 13.3 us).
   a.n_splits = dec_splits(B, Hkv, Tkv);
+  const bool single = group <= 2 && a.n_splits > 1 && Tkv * D <= 65536;
+  if (single) a.n_splits = 1;
   const int step = kDecWaves * (64 / (int)(D / 8));
   a.chunk = (int)(cdiv(cdiv(Tkv, a.n_splits), step) * step);
   a.sl2 = (float)(1.0 / sqrt((double)D)) * kLog2e;
@@ -3264,14 +3495,16 @@ int decode_launch(const void* q, const void* k, const void* v, void* o, float* l
   const int64_t blocks = B * Hkv * a.n_splits;
   if (blocks >= ((int64_t)1 << 31)) return fail(TRI_EINVAL, "attention decode: grid too large");
   hipStream_t st = (hipStream_t)stream;
-#define TRI_DEC_LAUNCH(TT, DD, GG) \
-  attn_decode_kernel<TT, DD, GG><<<(unsigned)blocks, 64 * kDecWaves, 0, st>>>(a)
-#define TRI_DEC_GROUPS(TT, DD)                        \
-  do {                                                \
-    if (group == 1) TRI_DEC_LAUNCH(TT, DD, 1);        \
-    else if (group == 2) TRI_DEC_LAUNCH(TT, DD, 2);   \
-    else if (group <= 4) TRI_DEC_LAUNCH(TT, DD, 4);   \
-    else TRI_DEC_LAUNCH(TT, DD, 8);                   \
+#define TRI_DEC_LAUNCH(TT, DD, GG, WW) \
+  attn_decode_kernel<TT, DD, GG, WW><<<(unsigned)blocks, 64 * (WW), 0, st>>>(a)
+#define TRI_DEC_GROUPS(TT, DD)                                      \
+  do {                                                              \
+    if (group > 2)                                                  \
+      attn_decode_mfma<TT, DD><<<(unsigned)blocks, 64 * kDecMWaves, 0, st>>>(a); \
+    else if (group == 2 && single) TRI_DEC_LAUNCH(TT, DD, 2, 16);   \
+    else if (group == 2) TRI_DEC_LAUNCH(TT, DD, 2, kDecWaves);      \
+    else if (single) TRI_DEC_LAUNCH(TT, DD, 1, 16);                 \
+    else TRI_DEC_LAUNCH(TT, DD, 1, kDecWaves);                      \
   } while (0)
   if (dtype == kBF16) {
     if (D == 64) TRI_DEC_GROUPS(bf16_t, 64); else TRI_DEC_GROUPS(bf16_t, 128);

@@ -169,6 +169,12 @@ __device__ __forceinline__ void dma16(const void* g, uint32_t lds) {
                : "memory", "m0");
 }
 
+// dma16 with the nontemporal hint (data read once).
+__device__ __forceinline__ void dma16_nt(const void* g, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "s"(lds)
+               : "memory", "m0");
+}
+
 // dma16 with a wave-uniform 64-bit base and a 32-bit per-lane byte offset
 // (the scalar-base addressing form: no 64-bit address arithmetic per lane).
 __device__ __forceinline__ void dma16s(const void* base, uint32_t voff, uint32_t lds) {
@@ -176,7 +182,12 @@ __device__ __forceinline__ void dma16s(const void* base, uint32_t voff, uint32_t
                : "memory", "m0");
 }
 
-// Same with 4 bytes per lane: lane i's dword lands at LDS byte lds + 4 i.
+__device__ __forceinline__ void dma16s_nt(const void* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(base), "s"(lds)
+               : "memory", "m0");
+}
+
+// dma16 with 4 bytes per lane: lane i's dword lands at LDS byte lds + 4 i.
 __device__ __forceinline__ void dma4(const void* g, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds)
                : "memory", "m0");

@@ -308,3 +308,36 @@ def test_attention_fp32_unaligned_rows():
     o = tritium.attention(*x)
     eo, _ = oracle.attention.forward(*(np32(t) for t in x), True)
     assert_close(o, eo, 1e-5, 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize(("b", "h", "hkv", "kv_len"), [
+    (1, 3, 3, 1024), (1, 4, 2, 511), (2, 3, 3, 513), (9, 12, 12, 300),
+    (2, 12, 3, 65), (1, 8, 1, 700), (1, 12, 4, 1025), (2, 16, 4, 4100), (40, 32, 8, 96)])
+def test_attention_decode_routes(dtype, head_dim, b, h, hkv, kv_len):
+    # one or two heads per kv head and up to 64 K elements of keys: one launch of 16
+    # wavefronts; groups of 3 and more: the matrix-core kernel, whole and ragged 32-key tiles
+    k, v = (randn((b, hkv, kv_len + 5, head_dim), dtype, 80 + i)[:, :, :kv_len] for i in range(2))
+    q = randn((b, h, 1, head_dim), dtype, 82)
+    o = tritium.attention(q, k, v, is_causal=False)
+    eo, e_lse = oracle.attention.forward(np32(q), np32(k), np32(v), False)
+    assert_close(o, eo, 2e-2, 2e-2, "o")
+    from helion_amd.attention import _attention_forward
+    _, lse = _attention_forward(q, k, v, False)
+    assert_close(lse, e_lse, 1e-4, 1e-4, "lse")
+
+
+def test_attention_decode_infinite_value():
+    # an infinite value is an infinite output in its column, not a NaN (the split weights'
+    # lower terms multiply it by zero or by a negative number)
+    q, k = randn((1, 8, 1, 128), torch.bfloat16, 90), randn((1, 2, 3000, 128), torch.bfloat16, 91)
+    v = randn((1, 2, 3000, 128), torch.bfloat16, 92)
+    v[0, 1, 1234, 7] = float("inf")
+    o = tritium.attention(q, k, v, is_causal=False)
+    assert torch.isinf(o[0, 4:, 0, 7]).all()
+    o[0, 4:, 0, 7] = 0
+    v[0, 1, 1234, 7] = 0
+    eo, _ = oracle.attention.forward(np32(q), np32(k), np32(v), False)
+    eo[0, 4:, 0, 7] = 0
+    assert_close(o, eo, 2e-2, 2e-2)
