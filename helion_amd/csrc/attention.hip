@@ -757,7 +757,9 @@ struct BtOffs {
 
 
 // ------------------------------------------------- MFMA forward, v2 (DMA) --
-// One workgroup = 8 wavefronts = 256 query rows of one (batch, head); each
+// One workgroup = 4 wavefronts = 128 query rows of one (batch, head), or 64
+// (SPLIT 2: two wavefronts share each 32-row block, taking the two 32-row
+// halves of every K/V tile, and merge their (m, l, O) at the end); each
 // wavefront owns 32 query rows (Q in registers) and computes, per 64-row K/V
 // tile, S^T = K Q^T (K fragments: 16-byte LDS reads) and O^T += V^T P^T
 // (V^T fragments: ds_read_b64_tr_b16 transposing reads of the row-major V
@@ -773,7 +775,7 @@ constexpr int kRing = 4;
 // K/V tiles in the LDS ring (3 measured 9% slower at the GPT block's shape)
 constexpr int kF2Stages = 2;
 
-template <typename T, int D>
+template <typename T, int D, int SPLIT>
 __global__ void __launch_bounds__(64 * kF2Waves, D > 128 ? 1 : 8 / kF2Waves)  // 2 wavefronts per SIMD (1 at D = 256)
 attn_fwd_v2(FwdArgs a) {
   typedef Mfma<T> M;
@@ -781,11 +783,14 @@ attn_fwd_v2(FwdArgs a) {
   typedef BTile<D> P;
   constexpr int KS = D / 16;
   constexpr int MT = D / 32;
+  constexpr int QB = kF2Waves / SPLIT;  // 32-row blocks per workgroup
+  constexpr int U = 2 / SPLIT;          // 32-key blocks of a tile per wavefront
   constexpr int STAGE = 2 * P::BYTES;  // K, V
   __shared__ __attribute__((aligned(1024))) char smem[kF2Stages * STAGE];
 
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int l32 = lane & 31, g = lane >> 5;
+  const int half = wave / QB;  // which 32 keys of every tile (SPLIT 2)
   int bh, rank;
   lpt_item(xcd_remap(blockIdx.x, gridDim.x), gridDim.x, a.B * a.H, a.n_tiles, a.causal, a.B * a.H,
            bh, rank);
@@ -796,8 +801,8 @@ attn_fwd_v2(FwdArgs a) {
   const T* kp = (const T*)a.k + b * a.sk_b + hk * a.sk_h;
   const T* vp = (const T*)a.v + b * a.sv_b + hk * a.sv_h;
   T* op = (T*)a.o + b * a.so_b + h * a.so_h;
-  const int q0 = qt * kF2BM;
-  const int qw0 = q0 + wave * 32;
+  const int q0 = qt * 32 * QB;
+  const int qw0 = q0 + (wave % QB) * 32;
   const int qrow = qw0 + l32;
   const bool qvalid = qrow < a.Tq;
   const float sl2 = a.scale * kLog2e;
@@ -818,7 +823,7 @@ attn_fwd_v2(FwdArgs a) {
   float m = -INFINITY, l = 0.f;
   float nm = 0.f;  // -m, or 0 while m is -inf (exp2 of a masked score is then 0)
 
-  const int kv_end = a.causal ? min(a.Tkv, q0 + kF2BM) : a.Tkv;
+  const int kv_end = a.causal ? min(a.Tkv, q0 + 32 * QB) : a.Tkv;
   const int n_kv = (int)cdiv(kv_end, kF2BN);
   // kF2Stages-deep ring: tile it + kF2Stages - 1 streams in while tile it
   // is multiplied, so a tile has kF2Stages - 1 tiles of compute to land
@@ -837,26 +842,30 @@ attn_fwd_v2(FwdArgs a) {
     if (it + kF2Stages - 1 < n_kv)
       dma.issue(smem + ((it + kF2Stages - 1) % kF2Stages) * STAGE, kp, a.sk_s, vp, a.sv_s,
                 kv0 + (kF2Stages - 1) * kF2BN, a.Tkv);
-    const char* Ks = smem + (it % kF2Stages) * STAGE;
+    const int kb = SPLIT == 2 ? kv0 + 32 * half : kv0;  // this wavefront's keys
+    const char* Ks = smem + (it % kF2Stages) * STAGE + (kb - kv0) * P::RB;
     const char* Vs = Ks + P::BYTES;
-    if (a.causal && kv0 > qw0 + 31) continue;  // this wavefront's rows see none of the tile
+    if (a.causal && kb > qw0 + 31) continue;  // this wavefront's rows see none of them
+    if (SPLIT == 2 && kb >= a.Tkv) continue;
 
-    // S^T = K Q^T: MFMA i = 2 st + u (the two 32-row halves interleaved);
+    // S^T = K Q^T: MFMA i = U st + u (the two 32-row halves interleaved);
     // each K fragment is read kRing MFMAs before its use, and the fences
     // keep the compiler from pulling reads back next to their MFMAs
-    auto kread = [&](int i) { return bt_row<T, D>(Ks, 32 * (i & 1), i >> 1); };
-    f32x16 s[2] = {zero16(), zero16()};
-    V kb[kRing];
+    auto kread = [&](int i) { return bt_row<T, D>(Ks, 32 * (i % U), i / U); };
+    f32x16 s[U];
 #pragma unroll
-    for (int i = 0; i < kRing; ++i) kb[i] = kread(i);
+    for (int u = 0; u < U; ++u) s[u] = zero16();
+    V kr[kRing];
+#pragma unroll
+    for (int i = 0; i < kRing; ++i) kr[i] = kread(i);
     // the MFMA chains run at raised wave priority, so the SIMD's arbiter
     // issues them ahead of the other wavefront's softmax (1.8% at head_dim 64)
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int i = 0; i < 2 * KS; ++i) {
+    for (int i = 0; i < U * KS; ++i) {
       sched_fence();
-      s[i & 1] = M::mma(kb[i % kRing], qf[i >> 1], s[i & 1]);
-      if (i + kRing < 2 * KS) kb[i % kRing] = kread(i + kRing);
+      s[i % U] = M::mma(kr[i % kRing], qf[i / U], s[i % U]);
+      if (i + kRing < U * KS) kr[i % kRing] = kread(i + kRing);
     }
     sched_fence();
     __builtin_amdgcn_s_setprio(0);
@@ -865,18 +874,18 @@ attn_fwd_v2(FwdArgs a) {
     V vb[kRing];
 #pragma unroll
     for (int i = 0; i < kRing; ++i) vb[i] = vread(i);
-    // s[u][r] = S^T[kv0 + 32u + 8(r/4) + 4g + r%4][qrow]; masked when that
+    // s[u][r] = S^T[kb + 32u + 8(r/4) + 4g + r%4][qrow]; masked when that
     // kv row is >= Tkv or (causal) > qrow
-    const bool need_mask = (kv0 + kF2BN > a.Tkv) || (a.causal && kv0 + kF2BN - 1 > qw0);
+    const bool need_mask = (kb + 32 * U > a.Tkv) || (a.causal && kb + 32 * U - 1 > qw0);
     if (need_mask) {
-      const int lim = (a.causal ? min(a.Tkv - 1, qrow) : a.Tkv - 1) - kv0 - 4 * g;
-      mask_above(s[0], lim);
-      mask_above(s[1], lim - 32);
+      const int lim = (a.causal ? min(a.Tkv - 1, qrow) : a.Tkv - 1) - kb - 4 * g;
+#pragma unroll
+      for (int u = 0; u < U; ++u) mask_above(s[u], lim - 32 * u);
     }
     // row max of the raw scores (the scale is positive), in log2 units
     float mx = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[u][r]);
     mx = xor32_max(mx) * sl2;
@@ -895,7 +904,7 @@ attn_fwd_v2(FwdArgs a) {
         for (int r = 0; r < 16; ++r) o[mt][r] *= alpha;
     }
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float p = fast_exp2(fmaf(s[u][r], sl2, nm));
@@ -909,7 +918,7 @@ attn_fwd_v2(FwdArgs a) {
     V pb;
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int i = 0; i < (kF2BN / 16) * MT; ++i) {
+    for (int i = 0; i < 2 * U * MT; ++i) {
       const int t = i / MT, mt = i % MT;
       sched_fence();
       if (mt == 0) {
@@ -917,13 +926,38 @@ attn_fwd_v2(FwdArgs a) {
         for (int j = 0; j < 8; ++j) pb[j] = (T)s[t >> 1][8 * (t & 1) + j];
       }
       o[mt] = M::mma(vb[i % kRing], pb, o[mt]);
-      if (i + kRing < (kF2BN / 16) * MT) vb[i % kRing] = vread(i + kRing);
+      if (i + kRing < 2 * U * MT) vb[i % kRing] = vread(i + kRing);
     }
     sched_fence();
     __builtin_amdgcn_s_setprio(0);
   }
 
-  const float lt = l + __shfl_xor(l, 32, 64);
+  float lt = l + __shfl_xor(l, 32, 64);
+  if constexpr (SPLIT == 2) {
+    // the second half's (m, l, o) through LDS, merged by the first
+    static_assert(QB * 64 * (16 * MT + 2) * 4 <= kF2Stages * STAGE, "merge buffer");
+    float* part = reinterpret_cast<float*>(smem) + (wave % QB) * 64 * (16 * MT + 2) + lane;
+    __syncthreads();
+    if (half == 1) {
+      part[0] = m;
+      part[64] = lt;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part[64 * (2 + 16 * mt + r)] = o[mt][r];
+    }
+    __syncthreads();
+    if (half == 1) return;
+    const float m1 = part[0], mm = fmaxf(m, m1);
+    const float w0 = m == -INFINITY ? 0.f : fast_exp2(m - mm);
+    const float w1 = m1 == -INFINITY ? 0.f : fast_exp2(m1 - mm);
+    m = mm;
+    lt = lt * w0 + part[64] * w1;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[mt][r] = o[mt][r] * w0 + part[64 * (2 + 16 * mt + r)] * w1;
+  }
   const float inv = lt > 0.f ? 1.0f / lt : 0.f;
   if (qvalid) {
     T* orow = op + (int64_t)qrow * a.so_s;
@@ -3038,6 +3072,30 @@ int simt_per_lane(int64_t d) {
     default: return fail(TRI_EINVAL, "attention: no MFMA kernel for head_dim %d", (int)d); \
   }
 
+// Whether the forward takes 64-row query tiles whose key sweep two
+// wavefronts share, instead of 128-row tiles (`blocks` of them, n_tiles a
+// head).  Twice the work items of half the length fill a grid that leaves
+// compute units idle, or whose longest causal sweeps set the time; the price
+// is twice the K/V stream into each CU per FLOP and a merge, which at
+// head_dim 128 costs 12 to 20% once the grid is full.  Measured (graph
+// replays, 128-row -> 64-row tiles, us):
+//   head_dim 128, causal  [1, 32, 512] 14.9 -> 12.4, [1, 12, 1024] 23.7 ->
+//     18.3, [1, 32, 1531] 37.5 -> 32.9, [1, 12, 4096] 104 -> 77, against
+//     [4, 32, 256] 11.3 -> 11.7, [3, 32, 384] 14.9 -> 16.0, [4, 32, 512]
+//     19.7 -> 24.7, [1, 32, 3000] 83 -> 94
+//   head_dim 128, no mask  [1, 16, 1000] 25.0 -> 19.1, against [2, 32, 500]
+//     17.3 -> 18.2, [1, 32, 1280] 40.6 -> 46.8
+//   head_dim 64  [1, 12, 1024] 17.3 -> 12.5, [2, 32, 768] 16.0 -> 13.0, [2,
+//     16, 2048] 33.2 -> 28.5, no mask [1, 32, 1280] 28.5 -> 24.5, against
+//     [8, 32, 256] 10.2 -> 11.4, [16, 16, 100] 6.2 -> 6.3, no mask [1, 16,
+//     4096] 85 -> 89
+bool split_forward(int64_t D, bool causal, int64_t n_tiles, int64_t blocks) {
+  int half_cus = 1;  // up to so many halves of the compute units in 128-row tiles
+  if (D == 64 && n_tiles > 1) half_cus = causal && n_tiles >= 4 ? 4 : 3;
+  if (D == 128 && causal) half_cus = n_tiles >= 8 ? 3 : n_tiles >= 4 ? 2 : 1;
+  return D <= 128 && 2 * blocks <= (int64_t)half_cus * cu_count();
+}
+
 template <typename T>
 int fwd_mfma(const FwdArgs& a, int64_t D, hipStream_t st) {
   // The ping-pong kernel (one 8-wavefront workgroup per CU, two 256-row
@@ -3057,13 +3115,20 @@ int fwd_mfma(const FwdArgs& a, int64_t D, hipStream_t st) {
   if (D == 64 || D == 128 || D == 256) {
     FwdArgs x = a;
     x.n_tiles = (int)cdiv(a.Tq, kF2BM);
-    const int64_t blocks = (int64_t)x.n_tiles * a.B * a.H;
-    if (D == 256)
-      attn_fwd_v2<T, 256><<<(unsigned)blocks, 64 * kF2Waves, 0, st>>>(x);
+    int64_t blocks = (int64_t)x.n_tiles * a.B * a.H;
+    if (split_forward(D, a.causal, x.n_tiles, blocks)) {
+      x.n_tiles = (int)cdiv(a.Tq, kF2BM / 2);
+      blocks = (int64_t)x.n_tiles * a.B * a.H;
+      if (D == 128)
+        attn_fwd_v2<T, 128, 2><<<(unsigned)blocks, 64 * kF2Waves, 0, st>>>(x);
+      else
+        attn_fwd_v2<T, 64, 2><<<(unsigned)blocks, 64 * kF2Waves, 0, st>>>(x);
+    } else if (D == 256)
+      attn_fwd_v2<T, 256, 1><<<(unsigned)blocks, 64 * kF2Waves, 0, st>>>(x);
     else if (D == 128)
-      attn_fwd_v2<T, 128><<<(unsigned)blocks, 64 * kF2Waves, 0, st>>>(x);
+      attn_fwd_v2<T, 128, 1><<<(unsigned)blocks, 64 * kF2Waves, 0, st>>>(x);
     else
-      attn_fwd_v2<T, 64><<<(unsigned)blocks, 64 * kF2Waves, 0, st>>>(x);
+      attn_fwd_v2<T, 64, 1><<<(unsigned)blocks, 64 * kF2Waves, 0, st>>>(x);
     return check_launch("attention forward (mfma)");
   }
   FwdArgs x = a;

@@ -341,3 +341,14 @@ def test_attention_decode_infinite_value():
     eo, _ = oracle.attention.forward(np32(q), np32(k), np32(v), False)
     eo[0, 4:, 0, 7] = 0
     assert_close(o, eo, 2e-2, 2e-2)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_forward_split_and_whole_tiles(head_dim, causal):
+    # small grids take 64-row query tiles whose two wavefronts a row block sweep alternate
+    # 32-key halves (a half without keys, without visible keys, ragged); large ones 128-row tiles
+    for tq, tkv in ((1, 31), (33, 33), (64, 96), (65, 97), (130, 64), (300, 40), (95, 128)):
+        _check(torch.float16, 1, 4, 2, tq, tkv, head_dim, causal, seed=100, grads=False)
+    _check(torch.bfloat16, 2, 3, 3, 257, 257, head_dim, causal, seed=101, layout="bthd")
+    _check_heads(torch.bfloat16, 8, 32, 8, 301, head_dim, causal, [(0, 0), (7, 7)], seed=102)
