@@ -352,3 +352,12 @@ def test_attention_forward_split_and_whole_tiles(head_dim, causal):
         _check(torch.float16, 1, 4, 2, tq, tkv, head_dim, causal, seed=100, grads=False)
     _check(torch.bfloat16, 2, 3, 3, 257, 257, head_dim, causal, seed=101, layout="bthd")
     _check_heads(torch.bfloat16, 8, 32, 8, 301, head_dim, causal, [(0, 0), (7, 7)], seed=102)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_attention_order_over_uneven_slices(dtype):
+    # causal grids whose slices do not divide over the 8 XCDs take their tiles rank by
+    # rank over all slices: block counts that are and are not multiples of 8, GQA
+    _check(dtype, 1, 12, 12, 260, 260, 64, True, seed=110)
+    _check(dtype, 3, 4, 2, 520, 520, 128, True, seed=111)
+    _check(dtype, 1, 20, 4, 390, 450, 64, True, seed=112)
