@@ -576,29 +576,72 @@ FwdLayout fwd_layout(int64_t N, int64_t V, int bm, int bn) {
   return L;
 }
 
-// K splits for an M x N product over K: the smallest power of two (at most 8,
-// at least 16 K tiles per split) whose grid fills the GPU twice; 1 for grids
-// that already do (config 4's dH and dW).
+// Splits that cutting K tiles into at most `s` ranges of equal length gives
+// (gemm_store's own rounding).
+int64_t even_splits(int64_t k_tiles, int64_t s) { return cdiv(k_tiles, cdiv(k_tiles, s)); }
+
+// Estimated microseconds of a product of `tiles` output tiles over k_tiles K
+// tiles cut into s ranges: whole rounds of one workgroup per compute unit, at
+// 1.8 us a K tile and 5 us a tile's fill and epilogue (the 768-wide products
+// below at full load), and the fp32 partials' write and read at 5 TB/s.
 template <typename T>
-int split_count(int64_t M, int64_t N, int64_t K) {
+double split_cost(int64_t tiles, int64_t k_tiles, int64_t s) {
   typedef CfgT<T> C;
-  const int64_t tiles = cdiv(M, C::BM) * cdiv(N, C::BN), target = 2 * (int64_t)cu_count();
-  int s = 1;
-  while (s < 8 && tiles * s < target && K / (2 * s) >= 16 * gemm::bk<C, T>()) s *= 2;
-  return s;
+  const double rounds = (double)cdiv(tiles * s, cu_count());
+  const double partials = s > 1 ? (double)(s * tiles) * (C::BM * C::BN * 8) / 5e6 : 0.0;
+  return rounds * (1.8 * (double)cdiv(k_tiles, s) + 5.0) + partials;
+}
+
+// K splits of `tiles` output tiles (at most 16, at least 16 K tiles each):
+// the cheapest by split_cost.  A power of two that filled the GPU twice left
+// 384 workgroups on 256 compute units for the 48 tiles of dH at 4091 x 768
+// (50257 rows reduced): 8 splits 429 us with their sum, 5 splits 342.
+template <typename T>
+int split_count(int64_t tiles, int64_t K) {
+  const int64_t kt = cdiv(K, gemm::bk<CfgT<T>, T>());
+  int64_t best = 1;
+  for (int64_t s = 2; s <= 16 && kt / s >= 16; ++s)
+    if (even_splits(kt, s) == s && split_cost<T>(tiles, kt, s) < split_cost<T>(tiles, kt, best))
+      best = s;
+  return (int)best;
+}
+
+// An M x N product over K as `body` rows (whole rounds of tiles, one pass)
+// and the other rows cut into `splits` K ranges: 591 tiles are 2.3 rounds of
+// 256 compute units, and a third round that is a third full costs as much as
+// a full one (dW [50257, 768] over 4091 tokens 369 -> 332 us).
+struct RowPlan {
+  int64_t body;
+  int splits;
+};
+template <typename T>
+RowPlan row_plan(int64_t M, int64_t N, int64_t K) {
+  typedef CfgT<T> C;
+  const int64_t kt = cdiv(K, gemm::bk<C, T>());
+  const int64_t tm = cdiv(M, C::BM), tn = cdiv(N, C::BN), cus = cu_count();
+  RowPlan best{0, split_count<T>(tm * tn, K)};
+  double cost = split_cost<T>(tm * tn, kt, best.splits);
+  const int64_t rounds = tm * tn / cus, body = rounds * cus / tn;
+  if (rounds > 0 && body > 0 && body < tm) {
+    const int64_t rest = (tm - body) * tn;
+    const int s = split_count<T>(rest, K);
+    const double c = split_cost<T>(body * tn, kt, 1) + split_cost<T>(rest, kt, s) + 5.0;
+    if (s > 1 && c < cost) best = RowPlan{body * C::BM, s};
+  }
+  return best;
 }
 
 struct BwdLayout {
   int64_t chunk, n_chunks, ld_g;
-  int sh, sw;  // K splits of the dH and dW products
+  int sh;  // K splits of dH
   size_t n_valid, gm, dh_acc, dw_part, total;
 };
 
 // The backward's workspace: the count of valid rows, G of one vocabulary
 // chunk [N, ld_g] (chunk rows chosen so that G fits kGBudget bytes, or
 // chunk_rows rounded up to the row tile), the fp32 dH accumulator [sh, N, D]
-// when there is more than one chunk or dH is split over K, and the fp32 dW
-// partials [sw, chunk, D] when dW is split.
+// when there is more than one chunk or dH is split over K, and the fp32
+// partials of the dW rows that are split over tokens.
 template <typename T>
 BwdLayout bwd_layout(int64_t N, int64_t D, int64_t V, bool need_dh, bool need_dw,
                      int64_t chunk_rows) {
@@ -619,12 +662,18 @@ BwdLayout bwd_layout(int64_t N, int64_t D, int64_t V, bool need_dh, bool need_dw
     off += (size_t)round_up((int64_t)bytes, 256);
     return at;
   };
-  L.sh = need_dh ? split_count<T>(N, D, std::min(chunk, V)) : 1;
-  L.sw = need_dw ? split_count<T>(std::min(chunk, V), D, N) : 1;
+  L.sh = need_dh ? split_count<T>(cdiv(N, CfgT<T>::BM) * cdiv(D, CfgT<T>::BN), std::min(chunk, V)) : 1;
+  // fp32 partials of dW's split rows, over the whole chunks and the last one
+  size_t dw_bytes = 0;
+  for (const int64_t vc : {std::min(chunk, V), V - (L.n_chunks - 1) * chunk}) {
+    const RowPlan p = row_plan<T>(vc, D, N);
+    if (need_dw && p.splits > 1)
+      dw_bytes = std::max(dw_bytes, (size_t)p.splits * (size_t)(vc - p.body) * D * 4);
+  }
   L.n_valid = take(4);
   L.gm = take((size_t)N * L.ld_g * esz);
   L.dh_acc = (need_dh && (L.n_chunks > 1 || L.sh > 1)) ? take((size_t)L.sh * N * D * 4) : 0;
-  L.dw_part = (need_dw && L.sw > 1) ? take((size_t)L.sw * std::min(chunk, V) * D * 4) : 0;
+  L.dw_part = dw_bytes > 0 ? take(dw_bytes) : 0;
   L.total = off;
   return L;
 }
@@ -735,15 +784,20 @@ int bwd_impl(const float* grad_out, const void* hidden, const void* weight, cons
     const T* wc = (const T*)weight + vc0 * D;
     if (need_dw) {
       // dW[vc0 : vc0 + vc, :] = G^T H: A[v][n] = G[n][v] and B[d][n] = H[n][d],
-      // both MN-contiguous; the token reduction in one product (or in sw
-      // fp32 partials summed in order), rounded once
-      gemm::Problem p{gm, hidden, L.ld_g, D, vc, D, N};
+      // both MN-contiguous; each row's token reduction in one product, or in
+      // fp32 partials summed in order, rounded once
+      const RowPlan plan = row_plan<T>(vc, D, N);
+      const int64_t whole = plan.splits > 1 ? plan.body : vc, rest = vc - whole;
       T* dst = (T*)dweight + vc0 * D;
-      if (L.sw == 1) {
+      if (whole > 0) {
+        gemm::Problem p{gm, hidden, L.ld_g, D, whole, D, N};
         if (int e = gemm_store<T, true, true>(p, nullptr, dst, false, D, st)) return e;
-      } else {
-        if (int e = gemm_store<T, true, true>(p, nullptr, dw_part, true, D, st, L.sw)) return e;
-        if (int e = tritium_sum_splits(dw_part, dst, L.sw, vc * D, std::is_same<T, bf16_t>::value ? kBF16 : kF16, st))
+      }
+      if (rest > 0) {
+        gemm::Problem p{gm + whole, hidden, L.ld_g, D, rest, D, N};
+        if (int e = gemm_store<T, true, true>(p, nullptr, dw_part, true, D, st, plan.splits)) return e;
+        if (int e = tritium_sum_splits(dw_part, dst + whole * D, plan.splits, rest * D,
+                                       std::is_same<T, bf16_t>::value ? kBF16 : kF16, st))
           return e;
       }
     }
