@@ -15,7 +15,7 @@
 // computes a BM x BN tile of C; wavefront (wm, wn) owns the (BM/WM) x (BN/WN)
 // sub-tile at (wm*BM/WM, wn*BN/WN), i.e. MT x NT tiles of 32 x 32.
 //
-// Accumulator layout (identical for the MFMA and the fp32 SIMT core, so the
+// Accumulator layout (identical for the 16-bit and the fp32 MFMA, so the
 // epilogues are shared): acc.t[i][j][r] holds
 //     C[m0 + acc_row(wm, i, r, g)][n0 + acc_col(wn, j, lane % 32)],  g = lane / 32,
 // the C layout of v_mfma_f32_32x32x16_{bf16,f16}.
@@ -42,6 +42,7 @@
 namespace tri {
 namespace gemm {
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -199,7 +200,7 @@ __device__ __forceinline__ void reg_tile(char* stage, const Problem& p, int64_t 
   }
 }
 
-// ---- per-K-tile compute: MFMA for 16-bit types, FMA for fp32 --------------
+// ---- per-K-tile compute: MFMA, 16-bit and fp32 ----------------------------
 __device__ __forceinline__ f32x16 mma(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
@@ -291,29 +292,28 @@ __device__ __forceinline__ void compute_tile(const char* stage, Acc<C>& acc, int
     mma_steps<C, T, Hook, 0, TA, TB>(As, Bs, acc, wm, wn, a, b, hook);
   } else {
     all_steps<C>(hook);  // no MFMA steps to spread over: the hook's work up front
-    // fp32: exact FMAs; one float4 (one granule) per row and per column per step
-#pragma unroll 1
-    for (int c = 0; c < C::GRAN; ++c) {
-      float4 b[C::NT];
+    // fp32: exact products and sums on v_mfma_f32_32x32x2_f32.  Lane half g
+    // reads granule 2 S + g of its row, so instruction e of a granule pair
+    // contracts k = 8 S + e and 8 S + 4 + e.  Against one FMA per element on
+    // the vector pipe (64 to 72 TFLOP/s, bound by the A reads that every row
+    // of the accumulators needed), [2048, 768] x 32000 forward and
+    // backward 4.31 -> 3.00 ms (the library products of the backward included)
+#pragma unroll
+    for (int S = 0; S < C::GRAN / 2; ++S) {
+      f32x4 a[C::MT], b[C::NT];
+#pragma unroll
+      for (int i = 0; i < C::MT; ++i)
+        a[i] = *reinterpret_cast<const f32x4*>(As + swz<C>(wm * C::WTM + 32 * i + l32, 2 * S + g));
 #pragma unroll
       for (int j = 0; j < C::NT; ++j)
-        b[j] = *reinterpret_cast<const float4*>(Bs + swz<C>(wn * C::WTN + 32 * j + l32, c));
+        b[j] = *reinterpret_cast<const f32x4*>(Bs + swz<C>(wn * C::WTN + 32 * j + l32, 2 * S + g));
 #pragma unroll
-      for (int i = 0; i < C::MT; ++i) {
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float4 a = *reinterpret_cast<const float4*>(As + swz<C>(acc_row<C>(wm, i, r, g), c));
+        for (int i = 0; i < C::MT; ++i)
 #pragma unroll
-          for (int j = 0; j < C::NT; ++j) {
-            float v = acc.t[i][j][r];
-            v = fmaf(a.x, b[j].x, v);
-            v = fmaf(a.y, b[j].y, v);
-            v = fmaf(a.z, b[j].z, v);
-            v = fmaf(a.w, b[j].w, v);
-            acc.t[i][j][r] = v;
-          }
-        }
-      }
+          for (int j = 0; j < C::NT; ++j)
+            acc.t[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][e], b[j][e], acc.t[i][j], 0, 0, 0);
     }
   }
 }
@@ -601,8 +601,8 @@ __device__ __forceinline__ void mainloop(const Problem& p, int tm, int tn, char*
 }
 
 // Configurations: 16-bit types run 256 x 256 tiles on 8 wavefronts (2 per
-// SIMD, 128 x 64 each), double-buffered 128-byte K rows; fp32 (exact SIMT
-// arithmetic) runs 128 x 128 tiles on 4 wavefronts.
+// SIMD, 128 x 64 each), double-buffered 128-byte K rows; fp32 runs
+// 128 x 128 tiles on 4 wavefronts.
 template <typename T> struct CfgOf { typedef Cfg<256, 256, 2, 4, 2, 128> type; };
 template <> struct CfgOf<float> { typedef Cfg<128, 128, 2, 2, 2> type; };
 
