@@ -8,14 +8,16 @@
 // instructions per product against about 16 * 6 VALU instructions: a plain
 // two-stage tile loop with two wavefronts per SIMD keeps the pipe busy.
 //
-// Tile and split: a workgroup owns 32 * RBLK rows of one (batch, head) --
-// query rows in the forward and dQ, kv rows in dK/dV -- and TWO wavefronts
-// share each 32-row block, taking the two 32-row halves of every streamed
-// 64-row tile; their partial results meet in LDS once, at the end, in a
-// fixed order.  A small batch of medium sequences (the usual fp32 call)
-// leaves few row tiles: 64-row tiles whose sweep is split over four
-// wavefronts keep every SIMD of a compute unit on the same short work item,
-// which balances causal sweeps better than 128-row tiles would.
+// Tile and split: a workgroup owns 64 rows of one (batch, head) (128 in the
+// head_dim 128 forward) -- query rows in the forward and dQ, kv rows in dK/dV
+// -- and SH wavefronts share each 32-row block, taking the 32-row parts of
+// every streamed step in turn; their partial results meet in LDS once, at the
+// end, in a fixed order.  A small batch of medium sequences (the usual fp32
+// call) leaves few row tiles, and causal ones of unequal length; short work
+// items balance best.  SH is 2 (64-row steps; two workgroups of four
+// wavefronts a CU at head_dim 64; at head_dim 128 eight wavefronts in the
+// forward and four, at 230 to 330 registers a lane, in the backward), or 4
+// where that leaves compute units idle (128-row steps, head_dim 64).
 //
 // Operands: a lane's own row (l32 = lane & 31) lives in registers as 16-byte
 // granules, elements 8 st + 4 g + j (g = lane >> 5); a tile's rows come from
@@ -129,31 +131,45 @@ __device__ __forceinline__ void f32_store_row(float* p, const f32x16 (&v)[D / 32
                     v[mt][4 * rr + 2] * sc, v[mt][4 * rr + 3] * sc);
 }
 
-// Two 64-row fp32 tiles by DMA (the 16-bit tiles' engine on rows of 2 D halves).
+// TILES pairs of 64-row fp32 tiles (rows r0.. of x and of y) by DMA, the
+// 16-bit tiles' engine on rows of 2 D halves.
 template <int D, int WAVES>
 struct F32Dma {
+  typedef BTile<2 * D> P;
   BtDma<bf16_t, 2 * D, WAVES> dma;
   __device__ __forceinline__ void init(int64_t sx, int64_t sy) { dma.init(2 * sx, 2 * sy); }
+  template <int TILES>
   __device__ __forceinline__ void issue(char* dst, const float* x, int64_t sx, const float* y,
                                         int64_t sy, int r0, int n_rows) const {
-    dma.issue(dst, (const bf16_t*)x, 2 * sx, (const bf16_t*)y, 2 * sy, r0, n_rows);
+#pragma unroll
+    for (int i = 0; i < TILES; ++i)
+      if (i == 0 || r0 + 64 * i < n_rows)
+        dma.issue(dst + i * 2 * P::BYTES, (const bf16_t*)x, 2 * sx, (const bf16_t*)y, 2 * sy,
+                  r0 + 64 * i, n_rows);
+  }
+  // byte offset of the i-th of SH 32-row blocks of x
+  template <int SH>
+  static __device__ __forceinline__ int rows_at(int i) {
+    if constexpr (SH == 2) return 32 * i * P::RB;
+    else return (i >> 1) * 2 * P::BYTES + (i & 1) * 32 * P::RB;
   }
 };
 
-// 32-row blocks per workgroup: the forward at head_dim 128 runs four (eight
-// wavefronts, two per SIMD beside its 128 KB of LDS); the backward kernels
-// at head_dim 128 hold 230 to 330 registers a lane and run one wavefront per
-// SIMD; everything at head_dim 64 runs two workgroups of four per CU.
+// Row blocks of 32 per workgroup; SH wavefronts (2 or 4) share each.
 template <int D> constexpr int f32_fwd_blocks() { return D == 128 ? 4 : 2; }
 constexpr int kF32BwdBlocks = 2;
+// workgroups per compute unit that the kernels are compiled for
+template <int D> constexpr int f32_groups(int waves) { return D == 64 && waves <= 4 ? 2 : 1; }
 
-template <int D>
-__global__ void __launch_bounds__(128 * f32_fwd_blocks<D>(), D == 128 ? 1 : 2)
+template <int D, int SH>
+__global__ void __launch_bounds__(64 * SH * f32_fwd_blocks<D>(), f32_groups<D>(SH * f32_fwd_blocks<D>()))
 attn_fwd_f32(FwdArgs a) {
-  constexpr int QB = f32_fwd_blocks<D>(), WAVES = 2 * QB, MT = D / 32, BM = 32 * QB;
+  constexpr int QB = f32_fwd_blocks<D>(), WAVES = SH * QB, MT = D / 32;
+  constexpr int BM = 32 * QB, BK = 32 * SH;  // rows, keys per step
   typedef BTile<2 * D> P;
-  constexpr int STAGE = 2 * P::BYTES;  // K, V
-  static_assert(QB * 64 * (16 * MT + 2) * 4 <= 2 * STAGE, "merge buffer");
+  constexpr int PART = QB * 64 * (16 * MT + 2);
+  constexpr int STAGE = SH * P::BYTES;  // K, V of every 64 keys
+  static_assert((SH - 1) * PART * 4 <= 2 * STAGE, "merge buffer");
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
 
   const int lane = threadIdx.x & 63, wave = wave_id();
@@ -179,18 +195,18 @@ attn_fwd_f32(FwdArgs a) {
   float m = -INFINITY, nm = 0.f, l = 0.f;  // nm: -m, 0 while m is -inf
 
   const int kv_end = a.causal ? min(a.Tkv, q0 + BM) : a.Tkv;
-  const int n_kv = (int)cdiv(kv_end, 64);
+  const int n_kv = (int)cdiv(kv_end, BK);
   F32Dma<D, WAVES> dma;
   dma.init(a.sk_s, a.sv_s);
-  if (n_kv > 0) dma.issue(smem, kp, a.sk_s, vp, a.sv_s, 0, a.Tkv);
+  if (n_kv > 0) dma.template issue<SH / 2>(smem, kp, a.sk_s, vp, a.sv_s, 0, a.Tkv);
   for (int it = 0; it < n_kv; ++it) {
     wait_vmcnt<0>();
     __syncthreads();
     if (it + 1 < n_kv)
-      dma.issue(smem + ((it + 1) & 1) * STAGE, kp, a.sk_s, vp, a.sv_s, 64 * (it + 1), a.Tkv);
-    const int kb = 64 * it + 32 * half;  // this wavefront's 32 keys
+      dma.template issue<SH / 2>(smem + ((it + 1) & 1) * STAGE, kp, a.sk_s, vp, a.sv_s, BK * (it + 1), a.Tkv);
+    const int kb = BK * it + 32 * half;  // this wavefront's 32 keys
     if (kb >= a.Tkv || (a.causal && kb > qw0 + 31)) continue;
-    const char* Ks = smem + (it & 1) * STAGE + 32 * half * P::RB;
+    const char* Ks = smem + (it & 1) * STAGE + F32Dma<D, WAVES>::template rows_at<SH>(half);
     const char* Vs = Ks + P::BYTES;
     f32x16 s = f32_rows<D>(of, Ks, qf, zero16());
     if (kb + 32 > a.Tkv || (a.causal && kb + 31 > qw0))
@@ -221,62 +237,72 @@ attn_fwd_f32(FwdArgs a) {
   }
   l += __shfl_xor(l, 32, 64);
 
-  // the second half's (m, l, o) into LDS, merged by the first
+  // the other wavefronts' (m, l, o) into LDS, merged by the first
   float* part = reinterpret_cast<float*>(smem) + qb * 64 * (16 * MT + 2) + lane;
   __syncthreads();
-  if (half == 1) {
-    part[0] = m;
-    part[64] = l;
+  if (half > 0) {
+    float* out = part + (half - 1) * PART;
+    out[0] = m;
+    out[64] = l;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) part[64 * (2 + 16 * mt + r)] = o[mt][r];
+      for (int r = 0; r < 16; ++r) out[64 * (2 + 16 * mt + r)] = o[mt][r];
   }
   __syncthreads();
-  if (half == 1 || !qvalid) return;
-  const float m1 = part[0], mt_ = fmaxf(m, m1);
-  const float w0 = m == -INFINITY ? 0.f : fast_exp2((m - mt_) * kLog2e);
-  const float w1 = m1 == -INFINITY ? 0.f : fast_exp2((m1 - mt_) * kLog2e);
-  l = l * w0 + part[64] * w1;
-  // no visible key: zeros; visible keys whose scores are all -inf: NaN, as exp(-inf + inf)
-  const float inv = l > 0.f ? 1.0f / l : (n_kv > 0 ? __builtin_nanf("") : 0.f);
+  if (half > 0 || !qvalid) return;
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[mt][r] = o[mt][r] * w0 + part[64 * (2 + 16 * mt + r)] * w1;
-  f32_store_row<D>((float*)a.o + b * a.so_b + h * a.so_h + (int64_t)qrow * a.so_s, o, inv, g);
-  if (g == 0)
-    a.lse[(int64_t)bh * a.Tq + qrow] = l > 0.f || n_kv == 0 ? mt_ + logf(l) : __builtin_nanf("");
-}
-
-// Sum of the two halves' accumulators: half 1 hands its over through LDS.
-template <int MT>
-__device__ __forceinline__ void f32_merge(float* part, f32x16 (&v)[MT], int half) {
-  __syncthreads();
-  if (half == 1) {
+  for (int i = 0; i < SH - 1; ++i, part += PART) {
+    const float m1 = part[0], mm = fmaxf(m, m1);
+    const float w0 = m == -INFINITY ? 0.f : fast_exp2((m - mm) * kLog2e);
+    const float w1 = m1 == -INFINITY ? 0.f : fast_exp2((m1 - mm) * kLog2e);
+    m = mm;
+    l = l * w0 + part[64] * w1;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) part[64 * (16 * mt + r)] = v[mt][r];
+      for (int r = 0; r < 16; ++r) o[mt][r] = o[mt][r] * w0 + part[64 * (2 + 16 * mt + r)] * w1;
+  }
+  // no visible key: zeros; visible keys whose scores are all -inf: NaN, as exp(-inf + inf)
+  const float inv = l > 0.f ? 1.0f / l : (n_kv > 0 ? __builtin_nanf("") : 0.f);
+  f32_store_row<D>((float*)a.o + b * a.so_b + h * a.so_h + (int64_t)qrow * a.so_s, o, inv, g);
+  if (g == 0)
+    a.lse[(int64_t)bh * a.Tq + qrow] = l > 0.f || n_kv == 0 ? m + logf(l) : __builtin_nanf("");
+}
+
+// Sum of the accumulators of the SH wavefronts of a row block, in order: the
+// others hand theirs to the first through LDS (PART floats apart).
+template <int MT, int SH, int PART>
+__device__ __forceinline__ void f32_merge(float* part, f32x16 (&v)[MT], int half) {
+  __syncthreads();
+  if (half > 0) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) part[(half - 1) * PART + 64 * (16 * mt + r)] = v[mt][r];
   }
   __syncthreads();
   if (half == 0) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int i = 0; i < SH - 1; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) v[mt][r] += part[64 * (16 * mt + r)];
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[mt][r] += part[i * PART + 64 * (16 * mt + r)];
   }
 }
 
 // dQ, and delta = rowsum(dO * O) for the dK/dV kernel: S^T = K Q^T and
 // dP^T = V dO^T from row reads, dQ^T += K^T dS^T.
-template <int D>
-__global__ void __launch_bounds__(128 * kF32BwdBlocks, D == 128 ? 1 : 2)
+template <int D, int SH>
+__global__ void __launch_bounds__(64 * SH * kF32BwdBlocks, f32_groups<D>(SH * kF32BwdBlocks))
 attn_bwd_dq_f32(BwdArgs a) {
-  constexpr int QB = kF32BwdBlocks, WAVES = 2 * QB, MT = D / 32, BM = 32 * QB;
+  constexpr int QB = kF32BwdBlocks, WAVES = SH * QB, MT = D / 32;
+  constexpr int BM = 32 * QB, BK = 32 * SH;
   typedef BTile<2 * D> P;
-  constexpr int STAGE = 2 * P::BYTES;  // K, V
-  static_assert(QB * 64 * 16 * MT * 4 <= 2 * STAGE, "merge buffer");
+  constexpr int PART = QB * 64 * 16 * MT;
+  constexpr int STAGE = SH * P::BYTES;  // K, V of every 64 keys
+  static_assert((SH - 1) * PART * 4 <= 2 * STAGE, "merge buffer");
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
 
   const int lane = threadIdx.x & 63, wave = wave_id();
@@ -315,18 +341,18 @@ attn_bwd_dq_f32(BwdArgs a) {
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) dq[mt] = zero16();
   const int kv_end = a.causal ? min(a.Tkv, q0 + BM) : a.Tkv;
-  const int n_kv = (int)cdiv(kv_end, 64);
+  const int n_kv = (int)cdiv(kv_end, BK);
   F32Dma<D, WAVES> dma;
   dma.init(a.sk_s, a.sv_s);
-  if (n_kv > 0) dma.issue(smem, kp, a.sk_s, vp, a.sv_s, 0, a.Tkv);
+  if (n_kv > 0) dma.template issue<SH / 2>(smem, kp, a.sk_s, vp, a.sv_s, 0, a.Tkv);
   for (int it = 0; it < n_kv; ++it) {
     wait_vmcnt<0>();
     __syncthreads();
     if (it + 1 < n_kv)
-      dma.issue(smem + ((it + 1) & 1) * STAGE, kp, a.sk_s, vp, a.sv_s, 64 * (it + 1), a.Tkv);
-    const int kb = 64 * it + 32 * half;
+      dma.template issue<SH / 2>(smem + ((it + 1) & 1) * STAGE, kp, a.sk_s, vp, a.sv_s, BK * (it + 1), a.Tkv);
+    const int kb = BK * it + 32 * half;
     if (kb >= a.Tkv || (a.causal && kb > qw0 + 31)) continue;
-    const char* Ks = smem + (it & 1) * STAGE + 32 * half * P::RB;
+    const char* Ks = smem + (it & 1) * STAGE + F32Dma<D, WAVES>::template rows_at<SH>(half);
     const char* Vs = Ks + P::BYTES;
     f32x16 s = f32_rows<D>(of, Ks, qf, zero16());
     const f32x16 dp = f32_rows<D>(of, Vs, df, zero16());
@@ -337,20 +363,23 @@ attn_bwd_dq_f32(BwdArgs a) {
       s[r] = fast_exp2(fmaf(s[r], a.scale, -lse) * kLog2e) * (dp[r] - dl);
     f32_cols<D>(of, Ks, s, dq);
   }
-  f32_merge<MT>(reinterpret_cast<float*>(smem) + qb * 64 * 16 * MT + lane, dq, half);
+  f32_merge<MT, SH, PART>(reinterpret_cast<float*>(smem) + qb * 64 * 16 * MT + lane, dq, half);
   if (half == 0 && qvalid)
     f32_store_row<D>((float*)a.dq + b * a.sdq_b + h * a.sdq_h + (int64_t)qrow * a.sdq_s, dq, a.scale, g);
 }
 
 // dK and dV: a lane owns one kv row, the query tiles of every head of its
 // group stream by: S = Q K^T, dP = dO V^T, dV^T += dO^T P, dK^T += Q^T dS.
-template <int D>
-__global__ void __launch_bounds__(128 * kF32BwdBlocks, D == 128 ? 1 : 2)
+template <int D, int SH>
+__global__ void __launch_bounds__(64 * SH * kF32BwdBlocks, f32_groups<D>(SH * kF32BwdBlocks))
 attn_bwd_dkdv_f32(BwdArgs a) {
-  constexpr int KB = kF32BwdBlocks, WAVES = 2 * KB, MT = D / 32, BN = 32 * KB;
+  constexpr int KB = kF32BwdBlocks, WAVES = SH * KB, MT = D / 32;
+  constexpr int BN = 32 * KB, BQ = 32 * SH;  // kv rows, query rows per step
   typedef BTile<2 * D> P;
-  constexpr int STAGE = 2 * P::BYTES + 512;  // Q, dO, lse[64], delta[64]
-  static_assert(KB * 64 * 16 * MT * 4 <= 2 * STAGE && WAVES >= 2, "merge buffer");
+  constexpr int PART = KB * 64 * 16 * MT;
+  // Q and dO of every 64 query rows, then lse and delta (BQ floats each)
+  constexpr int STAGE = SH * P::BYTES + SH * 256;
+  static_assert((SH - 1) * PART * 4 <= 2 * STAGE && WAVES >= SH, "merge buffer");
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
 
   const int lane = threadIdx.x & 63, wave = wave_id();
@@ -373,17 +402,19 @@ attn_bwd_dkdv_f32(BwdArgs a) {
   for (int mt = 0; mt < MT; ++mt) dk[mt] = dv[mt] = zero16();
 
   const int q_begin = a.causal ? kv0 : 0;  // top-left causal: rows < kv0 see none
-  const int n_q = a.Tq > q_begin ? (int)cdiv(a.Tq - q_begin, 64) : 0;
+  const int n_q = a.Tq > q_begin ? (int)cdiv(a.Tq - q_begin, BQ) : 0;
   const int n_steps = n_q * group;
   F32Dma<D, WAVES> dma;
   dma.init(a.sq_s, a.sdo_s);
   auto issue = [&](int hq, int q0, char* stage) {
-    dma.issue(stage, (const float*)a.q + b * a.sq_b + hq * a.sq_h, a.sq_s,
-              (const float*)a.dout + b * a.sdo_b + hq * a.sdo_h, a.sdo_s, q0, a.Tq);
-    const int64_t row = ((int64_t)b * a.H + hq) * a.Tq + min(q0 + lane, a.Tq - 1);
-    if (wave == 0) dma4(a.lse + row, __builtin_amdgcn_readfirstlane(lds_addr(stage + 2 * P::BYTES)));
-    if (wave == 1)
-      dma4(a.delta + row, __builtin_amdgcn_readfirstlane(lds_addr(stage + 2 * P::BYTES + 256)));
+    dma.template issue<SH / 2>(stage, (const float*)a.q + b * a.sq_b + hq * a.sq_h, a.sq_s,
+                               (const float*)a.dout + b * a.sdo_b + hq * a.sdo_h, a.sdo_s, q0, a.Tq);
+    // wavefront 2 i: lse of 64-row tile i, 2 i + 1: delta
+    const int64_t row = ((int64_t)b * a.H + hq) * a.Tq + min(q0 + 64 * (wave >> 1) + lane, a.Tq - 1);
+    if (wave < SH)
+      dma4((wave & 1 ? a.delta : a.lse) + row,
+           __builtin_amdgcn_readfirstlane(
+               lds_addr(stage + SH * P::BYTES + (wave & 1) * SH * 128 + (wave >> 1) * 256)));
   };
   // (head, tile) of the current step and of the one being fetched
   int hq = hk * group, qi = 0, hq_n = hq, qi_n = 0;
@@ -397,13 +428,13 @@ attn_bwd_dkdv_f32(BwdArgs a) {
       qi_n = 0;
       ++hq_n;
     }
-    if (step + 1 < n_steps) issue(hq_n, q_begin + 64 * qi_n, smem + ((step + 1) & 1) * STAGE);
-    const int qb = q_begin + 64 * qi + 32 * half;  // this wavefront's 32 query rows
+    if (step + 1 < n_steps) issue(hq_n, q_begin + BQ * qi_n, smem + ((step + 1) & 1) * STAGE);
+    const int qb = q_begin + BQ * qi + 32 * half;  // this wavefront's 32 query rows
     if (qb >= a.Tq || (a.causal && qb + 31 < kvb)) continue;
     const char* stage = smem + (step & 1) * STAGE;
-    const char* Qs = stage + 32 * half * P::RB;
+    const char* Qs = stage + F32Dma<D, WAVES>::template rows_at<SH>(half);
     const char* dOs = Qs + P::BYTES;
-    const float* lse_s = reinterpret_cast<const float*>(stage + 2 * P::BYTES) + 32 * half + 4 * g;
+    const float* lse_s = reinterpret_cast<const float*>(stage + SH * P::BYTES) + 32 * half + 4 * g;
     f32x16 s = f32_rows<D>(of, Qs, kf, zero16());
     f32x16 dp = f32_rows<D>(of, dOs, vf, zero16());
     if ((a.causal && qb < kvb + 31) || qb + 32 > a.Tq)
@@ -411,7 +442,7 @@ attn_bwd_dkdv_f32(BwdArgs a) {
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) {
       const float4 L = *reinterpret_cast<const float4*>(lse_s + 8 * rr);
-      const float4 Dl = *reinterpret_cast<const float4*>(lse_s + 64 + 8 * rr);
+      const float4 Dl = *reinterpret_cast<const float4*>(lse_s + BQ + 8 * rr);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int r = 4 * rr + j;
@@ -423,12 +454,24 @@ attn_bwd_dkdv_f32(BwdArgs a) {
     f32_cols<D>(of, Qs, dp, dk);
   }
   float* part = reinterpret_cast<float*>(smem) + blk * 64 * 16 * MT + lane;
-  f32_merge<MT>(part, dk, half);
-  f32_merge<MT>(part, dv, half);
+  f32_merge<MT, SH, PART>(part, dk, half);
+  f32_merge<MT, SH, PART>(part, dv, half);
   if (half == 0 && kvvalid) {
     f32_store_row<D>((float*)a.dk + b * a.sdk_b + hk * a.sdk_h + (int64_t)kvw * a.sdk_s, dk, a.scale, g);
     f32_store_row<D>((float*)a.dv + b * a.sdv_b + hk * a.sdv_h + (int64_t)kvw * a.sdv_s, dv, 1.f, g);
   }
+}
+
+// Whether four wavefronts share a row block (head_dim 64): `blocks` of 64
+// rows that leave compute units idle, or under the causal mask at most two of
+// them a compute unit, whose longest sweeps set the time.  Forward and
+// backward, two -> four wavefronts a block: [1, 32, 1024] 240 -> 206 us,
+// [2, 16, 700] 155 -> 129, [1, 16, 2048] 453 -> 362, against [4, 12, 1024]
+// 288 -> 326, [16, 12, 300] 154 -> 201 and, without a mask, [2, 12, 1024]
+// 309 -> 340: a compute unit then runs one workgroup whose wavefronts meet
+// at every barrier instead of two that cover each other.
+bool f32_share4(int64_t D, bool causal, int64_t blocks) {
+  return D == 64 && blocks <= (causal ? 2 : 1) * (int64_t)cu_count();
 }
 
 template <int D>
@@ -437,20 +480,34 @@ int fwd_f32(const FwdArgs& a, hipStream_t st) {
   constexpr int QB = f32_fwd_blocks<D>();
   x.n_tiles = (int)cdiv(a.Tq, 32 * QB);
   const int64_t blocks = (int64_t)x.n_tiles * a.B * a.H;
-  attn_fwd_f32<D><<<(unsigned)blocks, 128 * QB, 0, st>>>(x);
+  if constexpr (D == 64) {
+    if (f32_share4(D, a.causal, blocks)) {
+      attn_fwd_f32<D, 4><<<(unsigned)blocks, 256 * QB, 0, st>>>(x);
+      return check_launch("attention forward (fp32)");
+    }
+  }
+  attn_fwd_f32<D, 2><<<(unsigned)blocks, 128 * QB, 0, st>>>(x);
   return check_launch("attention forward (fp32)");
 }
 
 // dQ first: it also computes delta, which the dK/dV kernel reads.
 template <int D>
 int bwd_f32(const BwdArgs& a, hipStream_t st) {
+  constexpr int RB = kF32BwdBlocks;
   BwdArgs x = a;
-  x.n_tiles = (int)cdiv(a.Tq, 32 * kF32BwdBlocks);
+  x.n_tiles = (int)cdiv(a.Tq, 32 * RB);
   const int64_t q_blocks = (int64_t)x.n_tiles * a.B * a.H;
-  attn_bwd_dq_f32<D><<<(unsigned)q_blocks, 128 * kF32BwdBlocks, 0, st>>>(x);
+  const int64_t kv_blocks = cdiv(a.Tkv, 32 * RB) * a.B * a.Hkv;
+  const bool q4 = f32_share4(D, a.causal, q_blocks), kv4 = f32_share4(D, a.causal, kv_blocks);
+  if constexpr (D == 64) {
+    if (q4) attn_bwd_dq_f32<D, 4><<<(unsigned)q_blocks, 256 * RB, 0, st>>>(x);
+  }
+  if (!q4) attn_bwd_dq_f32<D, 2><<<(unsigned)q_blocks, 128 * RB, 0, st>>>(x);
   if (int e = check_launch("attention backward (dq, fp32)")) return e;
-  x.n_tiles = (int)cdiv(a.Tkv, 32 * kF32BwdBlocks);
-  const int64_t kv_blocks = (int64_t)x.n_tiles * a.B * a.Hkv;
-  attn_bwd_dkdv_f32<D><<<(unsigned)kv_blocks, 128 * kF32BwdBlocks, 0, st>>>(x);
+  x.n_tiles = (int)cdiv(a.Tkv, 32 * RB);
+  if constexpr (D == 64) {
+    if (kv4) attn_bwd_dkdv_f32<D, 4><<<(unsigned)kv_blocks, 256 * RB, 0, st>>>(x);
+  }
+  if (!kv4) attn_bwd_dkdv_f32<D, 2><<<(unsigned)kv_blocks, 128 * RB, 0, st>>>(x);
   return check_launch("attention backward (dk/dv, fp32)");
 }

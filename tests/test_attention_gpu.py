@@ -288,8 +288,8 @@ def test_attention_pingpong_grid():
 
 
 # fp32 at head_dim 64 and 128 runs the fp32 matrix kernels: 64-row tiles (128
-# query rows a workgroup in the head_dim 128 forward) swept in two 32-row
-# halves.  Edges: one row, rows and keys just over and under 32, 64 and 128,
+# query rows a workgroup in the head_dim 128 forward) swept by two wavefronts a
+# row block, or four (head_dim 64, small grids).  Edges: one row, rows and keys just over and under 32, 64 and 128,
 # a half without keys, Tq != Tkv under the top-left mask, GQA, strided module
 # views; the last, rows that are not 16-byte aligned, stays on the SIMT path.
 # Tolerance 1e-5: fp32 sums of at most 300 terms of order 1.
@@ -301,6 +301,13 @@ def test_attention_pingpong_grid():
     (4, 4, 2, 192, 192, "bthd"), (2, 8, 8, 257, 257, "bhtd")])
 def test_attention_fp32_matrix_kernels(b, h, hkv, tq, tkv, layout, causal, head_dim):
     _check(torch.float32, b, h, hkv, tq, tkv, head_dim, causal, seed=61, layout=layout)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_fp32_large_grid(causal):
+    # 640 row tiles: two wavefronts a row block at head_dim 64 (four below 257 or 513)
+    _check_heads(torch.float32, 8, 16, 16, 300, 64, causal, [(0, 0), (5, 3), (7, 15)], seed=75,
+                 grads=True)
 
 
 def test_attention_fp32_unaligned_rows():
