@@ -6,7 +6,7 @@
 // P = exp(s - lse), dP = dO v^T, D_i = rowsum(P dP), dS = P (dP - D_i),
 // dV = P^T dO, dQ = dS k * scale, dK = dS^T q * scale).
 //
-// bf16 / fp16 inputs with head_dim in {16, 32, 64, 128} run on the MFMA path
+// bf16 / fp16 inputs with head_dim in {16, 32, 64, 128, 256} run on the MFMA path
 // (v_mfma_f32_32x32x16_{bf16,f16}, fp32 accumulation):
 //
 //  forward   a wavefront computes S^T = K Q^T for its 32 query rows against a
@@ -14,7 +14,8 @@
 //            so each lane owns ONE query column: the online-softmax max needs a
 //            single lane^32 exchange and P^T feeds the next MFMA
 //            (O^T = V^T P^T) straight from registers, V^T by transposing LDS
-//            reads.  attn_fwd_v2: 4 wavefronts = 128 query rows per workgroup;
+//            reads.  attn_fwd_v2: 4 wavefronts = 128 query rows per workgroup
+//            (64 on small grids, two wavefronts to a row block);
 //            attn_fwd_pp (head_dim 128, large grids): 8 wavefronts in two
 //            groups on opposite MFMA / softmax phases, two 256-row query tiles
 //            per workgroup.
@@ -1528,7 +1529,9 @@ attn_bwd_dq_mfma(BwdArgs a) {
 // sweeps the 64-row query tiles of every query head of the GQA group that
 // can see them: S = Q K^T and dP = dO V^T from row reads of the Q / dO
 // tiles, dV^T += dO^T P and dK^T += Q^T dS from transposing reads.
-template <typename T, int D, int WAVES, int PASS = 0>
+// SPLIT 2 (small grids, split_backward): 16 * WAVES kv rows, two wavefronts
+// on each 32 of them, one for either half of every query tile.
+template <typename T, int D, int WAVES, int PASS = 0, int SPLIT = 1>
 __global__ void __launch_bounds__(64 * WAVES, D == 64 ? 8 / WAVES : 1)
 attn_bwd_dkdv_v2(BwdArgs a) {
   // PASS 0: dK and dV; 1: dV alone; 2: dK alone (head_dim 256, where the K
@@ -1540,7 +1543,8 @@ attn_bwd_dkdv_v2(BwdArgs a) {
   typedef BTile<D> P;
   constexpr int KS = D / 16;
   constexpr int MT = D / 32;
-  constexpr int BN = 32 * WAVES;
+  constexpr int KB = WAVES / SPLIT;  // 32-row blocks of kv rows
+  constexpr int BN = 32 * KB;
   constexpr int STAGE = 2 * P::BYTES + 512;  // Q, dO, lse[64], delta[64]
   static_assert(WAVES >= 2 && BN % 64 == 0, "waves");
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
@@ -1553,7 +1557,8 @@ attn_bwd_dkdv_v2(BwdArgs a) {
   const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
   const int group = a.H / a.Hkv;
   const int kv0 = kt * BN;
-  const int kvb = kv0 + wave * 32;
+  const int half = wave / KB;  // which 32 query rows of every tile (SPLIT 2)
+  const int kvb = kv0 + (wave % KB) * 32;
   const int kvw = kvb + l32;  // this lane's kv row (MFMA column)
   const bool kvvalid = kvw < a.Tkv;
   const T* kp = (const T*)a.k + b * a.sk_b + hk * a.sk_h;
@@ -1642,6 +1647,7 @@ attn_bwd_dkdv_v2(BwdArgs a) {
     if (step + 1 < n_steps) issue(smem + ((step + 1) & 1) * STAGE);
     q0 = q0 + 64 == q_end ? q_begin : q0 + 64;
     if (a.causal && q0 + 63 < kvb) continue;  // this wavefront's kv rows see none of the tile
+    if (SPLIT == 2 && ((a.causal && q0 + 32 * half + 31 < kvb) || q0 + 32 * half >= a.Tq)) continue;
     const char* Qs = smem + (step & 1) * STAGE;
     const char* dOs = Qs + P::BYTES;
     const float* lse_s = reinterpret_cast<const float*>(Qs + 2 * P::BYTES);
@@ -1649,7 +1655,8 @@ attn_bwd_dkdv_v2(BwdArgs a) {
     const bool need_mask = (a.causal && q0 < kvb + 31) || q0 + 64 > a.Tq;
 
 #pragma unroll
-    for (int mq = 0; mq < 2; ++mq) {
+    for (int i = 0; i < 2 / SPLIT; ++i) {
+      const int mq = SPLIT == 2 ? half : i;
       f32x16 s = zero16(), dp = zero16();
       if constexpr (DO_DK) {  // dP - delta accumulates from -delta
 #pragma unroll
@@ -1710,6 +1717,30 @@ attn_bwd_dkdv_v2(BwdArgs a) {
     }
   }
 
+  if constexpr (SPLIT == 2) {
+    // the second half's sums through LDS, added to the first's
+    static_assert(PASS == 0 && KB * 64 * 32 * MT * 4 <= 2 * STAGE, "merge buffer");
+    float* part = reinterpret_cast<float*>(smem) + (wave % KB) * 64 * 32 * MT + lane;
+    __syncthreads();
+    if (half == 1) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          part[64 * (32 * mt + r)] = dk[mt][r];
+          part[64 * (32 * mt + 16 + r)] = dv[mt][r];
+        }
+    }
+    __syncthreads();
+    if (half == 1) return;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        dk[mt][r] += part[64 * (32 * mt + r)];
+        dv[mt][r] += part[64 * (32 * mt + 16 + r)];
+      }
+  }
   if (kvvalid) {
     T* dkr = (T*)a.dk + b * a.sdk_b + hk * a.sdk_h + (int64_t)kvw * a.sdk_s;
     T* dvr = (T*)a.dv + b * a.sdv_b + hk * a.sdv_h + (int64_t)kvw * a.sdv_s;
@@ -2153,7 +2184,9 @@ __device__ __forceinline__ void store_dq_row(f32x16 (&dq)[D / 32], T* dqr, float
 // wavefront 32 of them (Q, dO fragments in registers, lane = query row),
 // and sweeps the 64-row K/V tiles it can see: S^T = K Q^T and
 // dP^T = V dO^T from row reads, dQ^T += K^T dS^T from transposing reads.
-template <typename T, int D, int WAVES>
+// SPLIT 2 (small grids, split_backward): 16 * WAVES query rows, two
+// wavefronts on each 32 of them, one for either half of every K/V tile.
+template <typename T, int D, int WAVES, int SPLIT = 1>
 __global__ void __launch_bounds__(64 * WAVES, D > 128 ? 1 : 8 / WAVES)  // 2 wavefronts per SIMD (1 at D = 256)
 attn_bwd_dq_v2(BwdArgs a) {
   typedef Mfma<T> M;
@@ -2161,7 +2194,9 @@ attn_bwd_dq_v2(BwdArgs a) {
   typedef BTile<D> P;
   constexpr int KS = D / 16;
   constexpr int MT = D / 32;
-  constexpr int BM = 32 * WAVES;
+  constexpr int QB = WAVES / SPLIT;  // 32-row blocks of query rows
+  constexpr int U = 2 / SPLIT;       // 32-key blocks of a tile per wavefront
+  constexpr int BM = 32 * QB;
   constexpr int STAGE = 2 * P::BYTES;  // K, V
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
 
@@ -2178,7 +2213,8 @@ attn_bwd_dq_v2(BwdArgs a) {
   const T* kp = (const T*)a.k + b * a.sk_b + hk * a.sk_h;
   const T* vp = (const T*)a.v + b * a.sv_b + hk * a.sv_h;
   const int q0 = qt * BM;
-  const int qw0 = q0 + wave * 32;
+  const int half = wave / QB;  // which 32 keys of every tile (SPLIT 2)
+  const int qw0 = q0 + (wave % QB) * 32;
   const int qrow = qw0 + l32;
   const bool qvalid = qrow < a.Tq;
   const float sl2 = a.scale * kLog2e;
@@ -2197,8 +2233,10 @@ attn_bwd_dq_v2(BwdArgs a) {
     rpos_ok = rope_position(a.rope, b, a.Tq, qrow, rpos);
     rope_q_frag<T, D>(qf, a.rope, rpos, rpos_ok, g);
     T* qr = (T*)a.q_rot + ((int64_t)bh * a.Tq + qrow) * D;
+    if (half == 0) {
 #pragma unroll
-    for (int s = 0; s < KS; ++s) *reinterpret_cast<V*>(qr + 16 * s + 8 * g) = qf[s];
+      for (int s = 0; s < KS; ++s) *reinterpret_cast<V*>(qr + 16 * s + 8 * g) = qf[s];
+    }
   }
   const float lse2 = qvalid ? a.lse[(int64_t)bh * a.Tq + qrow] * kLog2e : INFINITY;
   // delta = rowsum(dO * O) for this lane's query row (the two lanes of a row
@@ -2214,7 +2252,7 @@ attn_bwd_dq_v2(BwdArgs a) {
     }
   }
   dl += __shfl_xor(dl, 32, 64);
-  if (qvalid && g == 0) a.delta[(int64_t)bh * a.Tq + qrow] = dl;
+  if (qvalid && g == 0 && half == 0) a.delta[(int64_t)bh * a.Tq + qrow] = dl;
 
   f32x16 dq[MT];
 #pragma unroll
@@ -2238,24 +2276,26 @@ attn_bwd_dq_v2(BwdArgs a) {
     __syncthreads();
     if (it + 1 < n_kv)
       dma.issue(smem + ((it + 1) & 1) * STAGE, kp, a.sk_s, vp, a.sv_s, kv0 + 64, a.Tkv);
-    if (a.causal && kv0 > qw0 + 31) continue;  // this wavefront's rows see none of the tile
-    const char* Ks = smem + (it & 1) * STAGE;
+    const int kb = SPLIT == 2 ? kv0 + 32 * half : kv0;  // this wavefront's keys
+    if (a.causal && kb > qw0 + 31) continue;  // this wavefront's rows see none of them
+    if (SPLIT == 2 && kb >= a.Tkv) continue;
+    const char* Ks = smem + (it & 1) * STAGE + (SPLIT == 2 ? 32 * half * P::RB : 0);
     const char* Vs = Ks + P::BYTES;
-    const bool need_mask = kv0 + 64 > a.Tkv || (a.causal && kv0 + 63 > qw0);
+    const bool need_mask = kb + 32 * U > a.Tkv || (a.causal && kb + 32 * U - 1 > qw0);
 
-    V dsb[4];  // dS^T rounded to T as formed: operand t holds rows 16t + 4g + {0..3}, 16t + 8 + ...
+    V dsb[2 * U];  // dS^T rounded to T as formed: operand t holds rows 16t + 4g + {0..3}, 16t + 8 + ...
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       f32x16 s = zero16(), dp = zero16();
 #pragma unroll
       for (int st = 0; st < KS; ++st) {
         s = M::mma(bt_row<T, D>(Ks, 32 * u, st), qf[st], s);
         dp = M::mma(bt_row<T, D>(Vs, 32 * u, st), df[st], dp);
       }
-      // s[r] = S^T[kv0 + 32u + 8(r/4) + 4g + r%4][qrow]; masked scores -> -inf (p = 0):
+      // s[r] = S^T[kb + 32u + 8(r/4) + 4g + r%4][qrow]; masked scores -> -inf (p = 0):
       // kv rows >= Tkv or (causal) > qrow
       if (need_mask)
-        mask_above(s, (a.causal ? min(a.Tkv - 1, qrow) : a.Tkv - 1) - kv0 - 32 * u - 4 * g);
+        mask_above(s, (a.causal ? min(a.Tkv - 1, qrow) : a.Tkv - 1) - kb - 32 * u - 4 * g);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float p = fast_exp2(fmaf(s[r], sl2, -lse2));
@@ -2263,12 +2303,30 @@ attn_bwd_dq_v2(BwdArgs a) {
       }
     }
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < 2 * U; ++t) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) dq[mt] = M::mma(bt_tr<T, D>(Ks, 16 * t, mt), dsb[t], dq[mt]);
     }
   }
 
+  if constexpr (SPLIT == 2) {
+    // the second half's sums through LDS, added to the first's
+    static_assert(QB * 64 * 16 * MT * 4 <= 2 * STAGE, "merge buffer");
+    float* part = reinterpret_cast<float*>(smem) + (wave % QB) * 64 * 16 * MT + lane;
+    __syncthreads();
+    if (half == 1) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part[64 * (16 * mt + r)] = dq[mt][r];
+    }
+    __syncthreads();
+    if (half == 1) return;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dq[mt][r] += part[64 * (16 * mt + r)];
+  }
   if (qvalid)
     store_dq_row<T, D>(dq, (T*)a.dq + b * a.sdq_b + h * a.sdq_h + (int64_t)qrow * a.sdq_s, a.scale,
                        a.rope, rope, rpos, rpos_ok, g);
@@ -3237,6 +3295,29 @@ int bwd_ds(const BwdArgs& a, hipStream_t st) {
   return check_launch("attention backward (dq from stored ds)");
 }
 
+// Whether a backward kernel at head_dim 64 takes half-size workgroup tiles
+// (SPLIT 2: 64 rows, two wavefronts on each 32-row block).  n_tiles and
+// blocks count whole tiles of 128 rows; dQ is decided by its query tiles and
+// dK/dV by its kv tiles, so under GQA they may differ.  A small grid's time is
+// that of its longest tile, which the split halves; a full grid only reads
+// twice as many tiles (8 to 18% slower at [16, 12, 1024], [8, 32, 200]).  A
+// causal grid's workgroups are of all lengths, so more of them still leave
+// compute units idle at the end, the more so the longer the longest is.
+// Measured (forward and backward, graph replays, whole -> split, us):
+//   causal  [1, 12, 1024] 62.2 -> 48.0, [1, 8, 4096] 202 -> 155, [1, 32/8,
+//     1531] 195 -> 144, [8, 16, 200] 28.4 -> 26.1, [4, 12, 700] 51.5 -> 44.8,
+//     [8, 12, 512] 45.8 -> 43.9, [1, 16, 4096] 235 -> 204, against [16, 16,
+//     128] 24.8 -> 25.2, [2, 32, 900] 72.0 -> 72.3, [3, 20, 1500] 121 -> 129
+//   no mask  [1, 12, 1024] 60.5 -> 47.1, [1, 8, 4096] 214 -> 190, [8, 10, 384]
+//     35.8 -> 34.7, against [8, 16, 200] 30.2 -> 31.2, [4, 12, 700] 65.7 ->
+//     70.8, [2, 16, 2048] 177 -> 193
+bool split_backward(int64_t D, bool causal, int64_t n_tiles, int64_t blocks) {
+  int half_cus = 0;  // up to so many halves of the compute units
+  if (n_tiles > 1) half_cus = causal || n_tiles > 2 ? 2 : 1;
+  if (causal && n_tiles >= 4) half_cus = n_tiles >= 16 ? 4 : 3;
+  return D == 64 && 2 * blocks <= (int64_t)half_cus * cu_count();
+}
+
 // dQ first: it also computes delta, which the dK/dV kernel reads.
 template <typename T, int D>
 int bwd_v2(const BwdArgs& a, hipStream_t st) {
@@ -3246,8 +3327,19 @@ int bwd_v2(const BwdArgs& a, hipStream_t st) {
   }
   BwdArgs x = a;
   x.n_tiles = (int)cdiv(a.Tq, 32 * WQ);
-  const int64_t q_blocks = (int64_t)x.n_tiles * a.B * a.H;
-  attn_bwd_dq_v2<T, D, WQ><<<(unsigned)q_blocks, 64 * WQ, 0, st>>>(x);
+  int64_t q_blocks = (int64_t)x.n_tiles * a.B * a.H;
+  bool split = false;
+  if constexpr (D == 64) {
+    split = split_backward(D, a.causal, x.n_tiles, q_blocks);
+    if (split) {
+      x.n_tiles = (int)cdiv(a.Tq, 16 * WQ);
+      q_blocks = (int64_t)x.n_tiles * a.B * a.H;
+      attn_bwd_dq_v2<T, D, WQ, 2><<<(unsigned)q_blocks, 64 * WQ, 0, st>>>(x);
+    }
+  }
+  if (!split) {
+    attn_bwd_dq_v2<T, D, WQ><<<(unsigned)q_blocks, 64 * WQ, 0, st>>>(x);
+  }
   if (int e = check_launch("attention backward (dq, mfma)")) return e;
   if (a.rope.cos != nullptr) {  // dK/dV take the rotated q the dQ kernel wrote
     x.q = a.q_rot;
@@ -3264,7 +3356,15 @@ int bwd_v2(const BwdArgs& a, hipStream_t st) {
     return launch_dkdv_pair<T, D, false>(x, st);
   }
   x.n_tiles = (int)cdiv(a.Tkv, 32 * WK);
-  const int64_t kv_blocks = (int64_t)x.n_tiles * a.B * a.Hkv;
+  int64_t kv_blocks = (int64_t)x.n_tiles * a.B * a.Hkv;
+  if constexpr (D == 64) {
+    if (split_backward(D, a.causal, x.n_tiles, kv_blocks)) {
+      x.n_tiles = (int)cdiv(a.Tkv, 16 * WK);
+      kv_blocks = (int64_t)x.n_tiles * a.B * a.Hkv;
+      attn_bwd_dkdv_v2<T, D, WK, 0, 2><<<(unsigned)kv_blocks, 64 * WK, 0, st>>>(x);
+      return check_launch("attention backward (dk/dv, mfma)");
+    }
+  }
   if constexpr (D == 256) {  // dV, then dK: one pass does not fit the registers
     attn_bwd_dkdv_v2<T, D, WK, 1><<<(unsigned)kv_blocks, 64 * WK, 0, st>>>(x);
     if (int e = check_launch("attention backward (dv, mfma)")) return e;

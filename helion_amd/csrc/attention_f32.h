@@ -29,8 +29,8 @@
 // 32 columns of the same row-major tile.  Nothing is transposed and no
 // score leaves the registers.
 //
-// Measured at [4, 12, 1024, 64] causal, forward and backward: 289 us a pass
-// against 9520 us on the SIMT kernels (78 + 110 + 139 us of kernels in the
+// Measured at [4, 12, 1024, 64] causal, forward and backward: 290 us a pass
+// against 9520 us on the SIMT kernels (76 + 107 + 135 us of kernels in the
 // profiler against 2820 + 3374 + 3394), 87 to 99 TFLOP/s each on the blocks
 // they compute; error against float64 6.5e-7 against 8.0e-7.
 //

@@ -1,4 +1,4 @@
-"""Attention HIP kernels (MFMA bf16/fp16, SIMT fp32) vs the float64 oracle,
+"""Attention HIP kernels (MFMA and SIMT) vs the float64 oracle,
 mirroring the reference's tests/tritium/test_attention.py (head dims, GQA,
 non-causal, KV-cache decode, autograd) plus the module's strided layout, ragged
 lengths, q_len != kv_len and head_dim 128.  Tolerance: bf16/fp16 max-abs 2e-2
@@ -359,6 +359,17 @@ def test_attention_forward_split_and_whole_tiles(head_dim, causal):
         _check(torch.float16, 1, 4, 2, tq, tkv, head_dim, causal, seed=100, grads=False)
     _check(torch.bfloat16, 2, 3, 3, 257, 257, head_dim, causal, seed=101, layout="bthd")
     _check_heads(torch.bfloat16, 8, 32, 8, 301, head_dim, causal, [(0, 0), (7, 7)], seed=102)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_backward_split_and_whole_tiles(causal):
+    # small grids of more than one 128-row tile take 64-row workgroup tiles, two wavefronts a
+    # row block on alternate 32-row halves of the tiles they sweep (a half out of range, masked
+    # out, ragged); dQ and dK/dV decide separately, so one may split and the other not
+    for tq, tkv in ((129, 31), (129, 129), (161, 300), (300, 161), (192, 256), (130, 1), (33, 700)):
+        _check(torch.float16, 1, 4, 2, tq, tkv, 64, causal, seed=120)
+    _check(torch.bfloat16, 2, 3, 3, 417, 417, 64, causal, seed=121, layout="bthd")
+    _check(torch.bfloat16, 4, 32, 1, 140, 280, 64, causal, seed=122)  # no mask: dQ whole, dK/dV split
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
