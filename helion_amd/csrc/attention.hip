@@ -1779,6 +1779,9 @@ attn_bwd_dkdv_v2(BwdArgs a) {
 // landed by the end of 2s + 2 (first read in 2s + 3).
 // DS: role B also stores each dS tile (cast to T, as the dK MFMAs take it)
 // in the stored-dS layout, for attn_bwd_dq_ds; zero in kv rows >= Tkv.
+// SPLIT 2 (small grids, split_pairs): 64 kv rows, two pairs on each 32 of
+// them, one for either 32-row half of every query tile; their sums meet in
+// LDS at the end.
 constexpr int kPairWaves = 8;
 constexpr int kPairBN = 128;
 constexpr int kDkvPPStages = 3;
@@ -1792,7 +1795,7 @@ struct PairLds {
 
 // The work of one (batch * kv head, kv tile) item; smem and xch_all are the
 // workgroup's LDS (PairLds sizes).
-template <typename T, int D, bool DS>
+template <typename T, int D, bool DS, int SPLIT>
 __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, char* xch_all,
                                                int bhk, int kt) {
   typedef Mfma<T> M;
@@ -1809,8 +1812,12 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
   const bool role_b = wave >= 4;  // wave-uniform
   const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
   const int group = a.H / a.Hkv;
-  const int kv0 = kt * kPairBN;
-  const int kvb = kv0 + pair * 32;
+  constexpr int KB = 4 / SPLIT;  // 32-row blocks of kv rows, SPLIT pairs on each
+  constexpr int U = 2 / SPLIT;   // 32-row parts of a query tile per pair
+  const int half = SPLIT == 2 ? pair / KB : 0;  // SPLIT 2: which one
+  const int hoff = 32 * half;
+  const int kv0 = kt * 32 * KB;
+  const int kvb = kv0 + (pair % KB) * 32;
   const int kvw = kvb + l32;
   const bool kvvalid = kvw < a.Tkv;
   const float sl2 = a.scale * kLog2e;
@@ -1897,9 +1904,9 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
   // i = 2 st + mq).  One kRing-deep operand ring runs from the first chain
   // into the second; the caller has read the first kDkvRing T2 operands into
   // it already (before the phase barrier).
-  constexpr int N2 = 4 * MT, N1 = 2 * KS, NPART = 2 * PER;
+  constexpr int N2 = 2 * U * MT, N1 = U * KS, NPART = 2 * PER;
   static_assert(N2 % kDkvRing == 0 && N1 >= kDkvRing, "operand ring");
-  static_assert(2 * NPART <= N2 && 2 * NPART <= N1, "DMA slots");
+  static_assert(SPLIT == 2 || (2 * NPART <= N2 && 2 * NPART <= N1), "DMA slots");
   V ring[kDkvRing];
   auto pre_tr = [&](const TrBase& b2) {
 #pragma unroll
@@ -1909,35 +1916,37 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
   // first T1 operands (read even when T1 is not multiplied after: a branch
   // per MFMA costs more than the unused reads of a resident tile); with
   // inter the next tile's DMAs go out after its odd MFMAs
-  auto tr_chain = [&](bool inter, const TrBase& b2, const char* T1, const V (&op)[4]) {
+  auto tr_chain = [&](bool inter, const TrBase& b2, const char* T1, const V (&op)[2 * U]) {
 #pragma unroll
     for (int i = 0; i < N2; ++i) {
       sched_fence();
       acc[i % MT] = M::mma(ring[i % kDkvRing], op[i / MT], acc[i % MT]);
       const int n = i + kDkvRing;
       if (n < N2) ring[i % kDkvRing] = fo.rd_tr(b2, 16 * (n / MT), n % MT);
-      else ring[i % kDkvRing] = fo.rd_row(T1, 32 * ((n - N2) & 1), (n - N2) >> 1);
-      if ((i & 1) && i < 2 * NPART && inter) issue_part(i >> 1);
+      else ring[i % kDkvRing] = fo.rd_row(T1, 32 * ((n - N2) % U), (n - N2) / U);
+      if constexpr (SPLIT == 1) {
+        if ((i & 1) && i < 2 * NPART && inter) issue_part(i >> 1);
+      }
     }
   };
-  auto rows_chain = [&](const char* T1, f32x16 (&x)[2]) {
+  auto rows_chain = [&](const char* T1, f32x16 (&x)[U]) {
 #pragma unroll
     for (int i = 0; i < N1; ++i) {
       sched_fence();
-      x[i & 1] = M::mma(ring[i % kDkvRing], frag[i >> 1], i < 2 ? zero16() : x[i & 1]);
+      x[i % U] = M::mma(ring[i % kDkvRing], frag[i / U], i < U ? zero16() : x[i % U]);
       const int n = i + kDkvRing;
-      if (n < N1) ring[i % kDkvRing] = fo.rd_row(T1, 32 * (n & 1), n >> 1);
+      if (n < N1) ring[i % kDkvRing] = fo.rd_row(T1, 32 * (n % U), n / U);
     }
   };
   // dtr: tr_chain (the ring pre-read by the caller), drows: rows_chain;
   // inter: the next tile's DMAs interleaved with tr_chain (needs dtr)
   auto mfma_phase = [&](bool dtr, bool drows, bool inter, const TrBase& b2, const char* T1,
-                        const V (&op)[4], f32x16 (&x)[2]) {
+                        const V (&op)[2 * U], f32x16 (&x)[U]) {
     if (dtr) {
       tr_chain(inter, b2, T1, op);
     } else {
 #pragma unroll
-      for (int i = 0; i < kDkvRing; ++i) ring[i] = fo.rd_row(T1, 32 * (i & 1), i >> 1);
+      for (int i = 0; i < kDkvRing; ++i) ring[i] = fo.rd_row(T1, 32 * (i % U), i / U);
     }
     if (drows) rows_chain(T1, x);
     sched_fence();
@@ -1951,8 +1960,8 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
   }
   wait_vmcnt<0>();
   lds_barrier();
-  f32x16 x[2];
-  V op[4];  // MFMA operand: slice t = 2 mq + u holds query rows 16t + 4g + {0..3}, 16t + 8 + 4g + {0..3}
+  f32x16 x[U];
+  V op[2 * U];  // MFMA operand: slice t = 2 mq + u (SPLIT 2: mq = half) holds query rows 16t + 4g + {0..3}, 16t + 8 + 4g + {0..3}
   // per step s: q0 of s and s - 1, the LDS stage of s (s - 1 is the stage before it)
   int q0c = q_last, q0p = q_last, sc = 0;
   if (!role_b) {
@@ -1965,11 +1974,12 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
       // DMAs of tile s + 1 (into the stage of tile s - 2, whose last reads
       // were in half-step 2s - 1)
       const bool nxt = s + 1 < n_steps;
-      const bool inter = nxt && prev && ld_fast();
+      const bool inter = SPLIT == 1 && nxt && prev && ld_fast();
       if (nxt && !inter) issue_all();
       if (inter) issue_stats();
       __builtin_amdgcn_s_setprio(1);
-      mfma_phase(prev, cur, inter, fo.tr_base(smem + sp * STAGE + P::BYTES), stc, op, x);
+      mfma_phase(prev, cur, inter, fo.tr_base(smem + sp * STAGE + P::BYTES + hoff * P::RB),
+                 stc + hoff * P::RB, op, x);
       __builtin_amdgcn_s_setprio(0);
       if (nxt) advance();
       lds_barrier();
@@ -1978,16 +1988,16 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
         const float* lse_s = reinterpret_cast<const float*>(stc + 2 * P::BYTES);
         const bool need_mask = (a.causal && q0c < kvb + 31) || q0c + 64 > a.Tq;
 #pragma unroll
-        for (int mq = 0; mq < 2; ++mq) {
+        for (int mq = 0; mq < U; ++mq) {
           // x[mq][r] = S[q0 + 32mq + 8(r/4) + 4g + r%4][kvw]; masked scores -> -inf (P = 0):
           // query rows >= Tq or (causal) < kvw
           if (need_mask) {
-            const int base = q0c + 32 * mq + 4 * g;
+            const int base = q0c + hoff + 32 * mq + 4 * g;
             mask_outside(x[mq], a.causal ? kvw - base : -64, a.Tq - base);
           }
 #pragma unroll
           for (int rr = 0; rr < 4; ++rr) {
-            const float4 L = *reinterpret_cast<const float4*>(lse_s + 32 * mq + 8 * rr + 4 * g);
+            const float4 L = *reinterpret_cast<const float4*>(lse_s + hoff + 32 * mq + 8 * rr + 4 * g);
             const float lv[4] = {L.x, L.y, L.z, L.w};
             float4 pv;
             float* pf = reinterpret_cast<float*>(&pv);
@@ -2002,7 +2012,7 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
         }
         // dO_s landed long ago: the first dV operands of half-step 2s + 2
         // are read here, under the barrier wait
-        pre_tr(fo.tr_base(stc + P::BYTES));
+        pre_tr(fo.tr_base(stc + P::BYTES + hoff * P::RB));
       }
       wait_vmcnt<0>();  // tile s + 1 (issued in half-step 2s)
       lds_barrier();
@@ -2029,15 +2039,15 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
         float* l = reinterpret_cast<float*>(stc + 2 * P::BYTES);
         l[lane] *= kLog2e;
       }
-      const TrBase qb = fo.tr_base(stp);
+      const TrBase qb = fo.tr_base(stp + hoff * P::RB);
       if (prev) {
         const float* del_s = reinterpret_cast<const float*>(stp + 2 * P::BYTES + 256);
 #pragma unroll
-        for (int mq = 0; mq < 2; ++mq) {
+        for (int mq = 0; mq < U; ++mq) {
 #pragma unroll
           for (int rr = 0; rr < 4; ++rr) {
             const float4 pv = *reinterpret_cast<const float4*>(xch + ((mq * 4 + rr) * 64 + lane) * 16);
-            const float4 Dl = *reinterpret_cast<const float4*>(del_s + 32 * mq + 8 * rr + 4 * g);
+            const float4 Dl = *reinterpret_cast<const float4*>(del_s + hoff + 32 * mq + 8 * rr + 4 * g);
             const float pp[4] = {pv.x, pv.y, pv.z, pv.w}, dd[4] = {Dl.x, Dl.y, Dl.z, Dl.w};
 #pragma unroll
             for (int j = 0; j < 4; ++j)
@@ -2052,10 +2062,10 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
             T* dst = ds_lane + ((int64_t)(b * a.H + hq0 + hp) * a.ds_bh +
                                 (ds_row(a.causal, q0p >> 6, n_kvt) + ds_j) * 4096);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
+            for (int t = 0; t < 2 * U; ++t) {
               u32x4 u = __builtin_bit_cast(u32x4, op[t]);
               if (ds_tail && !kvvalid) u = u32x4{0u, 0u, 0u, 0u};
-              __builtin_nontemporal_store(u, reinterpret_cast<u32x4*>(dst + 512 * t));
+              __builtin_nontemporal_store(u, reinterpret_cast<u32x4*>(dst + 512 * (2 * half + t)));
             }
           }
         }
@@ -2063,7 +2073,7 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
       lds_barrier();
       // half-step 2s + 1: dK^T += Q_{s-1}^T dS_{s-1}, dP_s = dO_s V^T
       __builtin_amdgcn_s_setprio(1);
-      mfma_phase(prev, cur, false, qb, stc + P::BYTES, op, x);
+      mfma_phase(prev, cur, false, qb, stc + P::BYTES + hoff * P::RB, op, x);
       __builtin_amdgcn_s_setprio(0);
       lds_barrier();
       q0p = q0c;
@@ -2074,6 +2084,26 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
     }
   }
 
+  if constexpr (SPLIT == 2) {
+    // the second halves' sums through LDS (past the last step's reads), added
+    // to the first's
+    static_assert(4 * 64 * 16 * MT * 4 <= kDkvPPStages * STAGE, "merge buffer");
+    float* part =
+        reinterpret_cast<float*>(smem) + ((role_b ? KB : 0) + pair % KB) * 64 * 16 * MT + lane;
+    __syncthreads();
+    if (half == 1) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part[64 * (16 * mt + r)] = acc[mt][r];
+    }
+    __syncthreads();
+    if (half == 1) return;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[mt][r] += part[64 * (16 * mt + r)];
+  }
   if (kvvalid) {
     T* out = role_b ? (T*)a.dk + b * a.sdk_b + hk * a.sdk_h + (int64_t)kvw * a.sdk_s
                     : (T*)a.dv + b * a.sdv_b + hk * a.sdv_h + (int64_t)kvw * a.sdv_s;
@@ -2103,7 +2133,7 @@ __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, char* smem, cha
 // [8, 32, 2048, 128], 16 tiles per head for 32 workgroups, each workgroup
 // kept one tile index and the kernel ran 1.17-1.36 ms against 1.43-1.65 ms
 // for the twice larger [4, 32, 4096, 128]).
-template <typename T, int D, bool DS, bool PERSIST>
+template <typename T, int D, bool DS, bool PERSIST, int SPLIT = 1>
 __global__ void __launch_bounds__(64 * kPairWaves, 1)  // 2 wavefronts per SIMD
 attn_bwd_dkdv_pair(BwdArgs a) {
   __shared__ __attribute__((aligned(1024))) char smem[kDkvPPStages * PairLds<D>::STAGE];
@@ -2116,10 +2146,10 @@ attn_bwd_dkdv_pair(BwdArgs a) {
     const int n_work = per * n_pairs;
     for (int w = slot; w < n_work; w += slots) {
       const int j = w / n_pairs, t0 = w % n_pairs, t1 = a.n_tiles - 1 - t0;
-      dkdv_pair_item<T, D, DS>(a, smem, xch_all, x * per + j, t0);
+      dkdv_pair_item<T, D, DS, SPLIT>(a, smem, xch_all, x * per + j, t0);
       lds_barrier();  // every wavefront is done with the LDS before the next item's DMAs
       if (t1 != t0) {
-        dkdv_pair_item<T, D, DS>(a, smem, xch_all, x * per + j, t1);
+        dkdv_pair_item<T, D, DS, SPLIT>(a, smem, xch_all, x * per + j, t1);
         lds_barrier();
       }
     }
@@ -2127,7 +2157,7 @@ attn_bwd_dkdv_pair(BwdArgs a) {
     int bhk, kt;  // kt = 0 sees the most queries: heaviest first
     lpt_item(xcd_remap(blockIdx.x, gridDim.x), gridDim.x, a.B * a.Hkv, a.n_tiles, a.causal,
              a.B * a.Hkv, bhk, kt);
-    dkdv_pair_item<T, D, DS>(a, smem, xch_all, bhk, kt);
+    dkdv_pair_item<T, D, DS, SPLIT>(a, smem, xch_all, bhk, kt);
   }
 }
 
@@ -3249,19 +3279,44 @@ int fwd_simt(const FwdArgs& a, int64_t D, hipStream_t st) {
 // measured no faster at the GPT block's shape; dQ 7% slower).
 constexpr int kDkvWaves = 4, kDqWaves = 4;
 
-// The dK/dV pair kernel over x.n_tiles kv tiles of every (batch, kv head):
-// persistent (one workgroup per compute unit) when the (batch, kv head)s
-// split evenly over the XCDs and there are at least two items per compute
-// unit, else one workgroup per item.
+// Whether the dK/dV pair kernel takes 64 kv rows a workgroup (SPLIT 2, two
+// pairs on each 32 of them) instead of 128: n_tiles and items count whole
+// tiles.  One workgroup fills a compute unit and a split one takes about half
+// the time per step, so it pays while the doubled grid still fits the chip at
+// once, and under the causal mask, whose items are of all lengths, up to one
+// whole item per compute unit.  Measured (forward and backward, graph replays,
+// whole -> split, us, head_dim 128):
+//   causal  [1, 12, 1024] 81.4 -> 71.3, [1, 32/8, 1531] 240 -> 186, [8, 8, 200]
+//     38.9 -> 35.1, [1, 32/8, 3000] 484 -> 391, [2, 32/8, 2048] 388 -> 345,
+//     [1, 16, 2048] 143 -> 134, against [2, 16, 1500] 127 -> 142, [1, 32/8,
+//     8192] 2163 -> 2374
+//   no mask  [1, 32/8, 1531] 263 -> 210, [1, 16, 1000] 83.6 -> 74.1, against
+//     [4, 32/8, 700] 184 -> 213, [1, 32, 1024] 100 -> 109
+bool split_pairs(bool causal, int64_t n_tiles, int64_t items) {
+  const int half_cus = causal && n_tiles >= 4 ? 2 : 1;  // up to so many halves of the compute units
+  return 2 * items <= (int64_t)half_cus * cu_count();
+}
+
+// The dK/dV pair kernel over the kv tiles of every (batch, kv head): split
+// tiles on small grids (above), persistent (one workgroup per compute unit)
+// when the (batch, kv head)s split evenly over the XCDs and there are at
+// least two items per compute unit, else one workgroup per item.
 template <typename T, int D, bool DS>
-int launch_dkdv_pair(const BwdArgs& x, hipStream_t st) {
+int launch_dkdv_pair(const BwdArgs& a, hipStream_t st) {
+  BwdArgs x = a;
+  x.n_tiles = (int)cdiv(a.Tkv, kPairBN);
   const int64_t n_bhk = (int64_t)x.B * x.Hkv;
   const int64_t items = n_bhk * x.n_tiles;
   const int cus = cu_count();
-  if (n_bhk % kXcds == 0 && cus % kXcds == 0 && items >= 2 * (int64_t)cus)
+  if (split_pairs(a.causal, x.n_tiles, items)) {
+    x.n_tiles = (int)cdiv(a.Tkv, kPairBN / 2);
+    attn_bwd_dkdv_pair<T, D, DS, false, 2>
+        <<<(unsigned)(n_bhk * x.n_tiles), 64 * kPairWaves, 0, st>>>(x);
+  } else if (n_bhk % kXcds == 0 && cus % kXcds == 0 && items >= 2 * (int64_t)cus) {
     attn_bwd_dkdv_pair<T, D, DS, true><<<(unsigned)cus, 64 * kPairWaves, 0, st>>>(x);
-  else
+  } else {
     attn_bwd_dkdv_pair<T, D, DS, false><<<(unsigned)items, 64 * kPairWaves, 0, st>>>(x);
+  }
   return check_launch(DS ? "attention backward (dk/dv storing ds)"
                          : "attention backward (dk/dv, mfma pairs)");
 }
@@ -3283,7 +3338,6 @@ int bwd_ds(const BwdArgs& a, hipStream_t st) {
     x.sq_b = (int64_t)a.H * a.Tq * D;
   }
   static_assert(D == 128, "stored-dS backward: head_dim 128");
-  x.n_tiles = (int)cdiv(a.Tkv, kPairBN);
   if (int e = launch_dkdv_pair<T, D, true>(x, st)) return e;
   x.q = a.q;  // dQ from dS reads K and dS only; the row strides of q stay the caller's
   x.sq_s = a.sq_s;
@@ -3351,10 +3405,7 @@ int bwd_v2(const BwdArgs& a, hipStream_t st) {
   // for the same VALU work, and one wavefront doing both roles with its
   // K and V fragments (attn_bwd_dkdv_v2) measured faster there (0.27 vs
   // 0.30 ms at [16, 12, 1024, 64], 1.35 vs 1.60 ms at [4, 32, 4096, 64])
-  if constexpr (D == 128) {
-    x.n_tiles = (int)cdiv(a.Tkv, kPairBN);
-    return launch_dkdv_pair<T, D, false>(x, st);
-  }
+  if constexpr (D == 128) return launch_dkdv_pair<T, D, false>(x, st);
   x.n_tiles = (int)cdiv(a.Tkv, 32 * WK);
   int64_t kv_blocks = (int64_t)x.n_tiles * a.B * a.Hkv;
   if constexpr (D == 64) {

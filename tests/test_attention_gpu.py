@@ -370,6 +370,23 @@ def test_attention_backward_split_and_whole_tiles(causal):
         _check(torch.float16, 1, 4, 2, tq, tkv, 64, causal, seed=120)
     _check(torch.bfloat16, 2, 3, 3, 417, 417, 64, causal, seed=121, layout="bthd")
     _check(torch.bfloat16, 4, 32, 1, 140, 280, 64, causal, seed=122)  # no mask: dQ whole, dK/dV split
+    _check_heads(torch.bfloat16, 5, 20, 20, 300, 64, causal, [(0, 0), (4, 19)], seed=123,
+                 grads=True)  # whole tiles
+
+
+@pytest.mark.parametrize("stored", [True, False])
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_split_pairs(monkeypatch, causal, stored):
+    # head_dim 128, small grids: 64 kv rows a workgroup, two wavefront pairs a row block on
+    # alternate halves of every query tile (a half out of range, masked out, ragged), with
+    # and without the stored dS
+    if not stored:
+        monkeypatch.setattr(importlib.import_module("helion_amd.attention"), "DS_WORKSPACE_MAX_BYTES", 0)
+    for tq, tkv in ((1, 129), (31, 200), (33, 33), (129, 129), (161, 300), (300, 161), (192, 256)):
+        _check(torch.float16, 1, 4, 2, tq, tkv, 128, causal, seed=130)
+    _check(torch.bfloat16, 2, 3, 3, 417, 417, 128, causal, seed=131, layout="bthd")
+    _check_heads(torch.bfloat16, 5, 20, 20, 300, 128, causal, [(0, 0), (4, 19)], seed=132,
+                 grads=True)  # 300 whole tiles: neither split nor persistent
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
