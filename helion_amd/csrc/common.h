@@ -164,32 +164,41 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // Callers wait for it explicitly (wait_vmcnt before the barrier that
 // publishes the tile); VMEM operations the compiler does not see can only
 // make its own in-order vmcnt waits stricter.
+//
+// The compiler inserts no wait states inside inline assembly, so the two that
+// these loads need are written out: one between the write of M0 and the LDS
+// load (s_nop 0, or the move of the base), and five between a vector
+// instruction's write of an SGPR (v_readfirstlane of a base) and a memory
+// instruction that reads it -- none after a scalar move, so the scalar-base
+// form copies its base.
 __device__ __forceinline__ void dma16(const void* g, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds)
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds)
                : "memory", "m0");
 }
 
 // dma16 with the nontemporal hint (data read once).
 __device__ __forceinline__ void dma16_nt(const void* g, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "s"(lds)
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "s"(lds)
                : "memory", "m0");
 }
 
 // dma16 with a wave-uniform 64-bit base and a 32-bit per-lane byte offset
 // (the scalar-base addressing form: no 64-bit address arithmetic per lane).
 __device__ __forceinline__ void dma16s(const void* base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(lds)
-               : "memory", "m0");
+  const void* sbase;
+  asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0"
+               : "=s"(sbase) : "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
 }
 
 __device__ __forceinline__ void dma16s_nt(const void* base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(base), "s"(lds)
-               : "memory", "m0");
+  const void* sbase;
+  asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0 nt"
+               : "=s"(sbase) : "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
 }
 
 // dma16 with 4 bytes per lane: lane i's dword lands at LDS byte lds + 4 i.
 __device__ __forceinline__ void dma4(const void* g, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds)
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds)
                : "memory", "m0");
 }
 
