@@ -3010,11 +3010,10 @@ attn_decode_combine(DecArgs a) {
 // One wavefront per row; lane i owns head-dim entries i, i+64, ...
 constexpr int kSimtMaxPerLane = 16;  // head_dim <= 1024
 
+// One wavefront, one row (of B * H * Tq).
 template <typename T, int PL>
-__global__ void __launch_bounds__(64)
-attn_fwd_simt(FwdArgs a, int D) {
-  const int lane = threadIdx.x;
-  const int64_t row = blockIdx.x;
+__device__ __forceinline__ void simt_fwd_row(const FwdArgs& a, int D, int64_t row) {
+  const int lane = threadIdx.x & 63;
   const int qrow = (int)(row % a.Tq);
   const int64_t bh = row / a.Tq;
   const int b = (int)(bh / a.H), h = (int)(bh % a.H);
@@ -3064,9 +3063,13 @@ attn_fwd_simt(FwdArgs a, int D) {
 
 template <typename T, int PL>
 __global__ void __launch_bounds__(64)
-attn_bwd_dq_simt(BwdArgs a, int D) {
-  const int lane = threadIdx.x;
-  const int64_t row = blockIdx.x;
+attn_fwd_simt(FwdArgs a, int D) {
+  simt_fwd_row<T, PL>(a, D, blockIdx.x);
+}
+
+template <typename T, int PL>
+__device__ __forceinline__ void simt_dq_row(const BwdArgs& a, int D, int64_t row) {
+  const int lane = threadIdx.x & 63;
   const int qrow = (int)(row % a.Tq);
   const int64_t bh = row / a.Tq;
   const int b = (int)(bh / a.H), h = (int)(bh % a.H);
@@ -3115,9 +3118,14 @@ attn_bwd_dq_simt(BwdArgs a, int D) {
 
 template <typename T, int PL>
 __global__ void __launch_bounds__(64)
-attn_bwd_dkdv_simt(BwdArgs a, int D) {
-  const int lane = threadIdx.x;
-  const int64_t row = blockIdx.x;  // over B * Hkv * Tkv
+attn_bwd_dq_simt(BwdArgs a, int D) {
+  simt_dq_row<T, PL>(a, D, blockIdx.x);
+}
+
+// One wavefront, one kv row (of B * Hkv * Tkv).
+template <typename T, int PL>
+__device__ __forceinline__ void simt_dkdv_row(const BwdArgs& a, int D, int64_t row) {
+  const int lane = threadIdx.x & 63;
   const int kv = (int)(row % a.Tkv);
   const int64_t bhk = row / a.Tkv;
   const int b = (int)(bhk / a.Hkv), hk = (int)(bhk % a.Hkv);
@@ -3170,6 +3178,12 @@ attn_bwd_dkdv_simt(BwdArgs a, int D) {
       dvo[d] = from_f32<T>(dv[j]);
     }
   }
+}
+
+template <typename T, int PL>
+__global__ void __launch_bounds__(64)
+attn_bwd_dkdv_simt(BwdArgs a, int D) {
+  simt_dkdv_row<T, PL>(a, D, blockIdx.x);
 }
 
 #include "attention_f32.h"

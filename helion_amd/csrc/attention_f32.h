@@ -37,6 +37,12 @@
 // Numerics: every product, sum and weight is fp32; p = 2^((s * scale - m)
 // log2 e) with the difference formed before the conversion to log2 units, so
 // its error is that of exp(s * scale - m).
+//
+// Masked pairs of a partly masked 32 x 32 block are multiplied too, with a
+// weight of zero, and zero times an infinite or NaN element of the other
+// operand is NaN.  So a workgroup with masked pairs whose sums end in any NaN
+// takes its rows again with the SIMT code, which visits the visible pairs
+// only: what a hidden row holds never reaches the result.
 
 // Per-lane byte offsets into a BTile of D fp32 (2 D 16-bit) columns: row
 // granule 2 i + g of row l32 (i < 8; a granule 16 columns of 16 bytes on is
@@ -155,6 +161,21 @@ struct F32Dma {
   }
 };
 
+template <int MT>
+__device__ __forceinline__ bool f32_any_nan(const f32x16 (&v)[MT]) {
+  bool nan = false;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) nan |= v[mt][r] != v[mt][r];
+  return nan;
+}
+
+// Whether any lane of the workgroup says so (a scalar).
+__device__ __forceinline__ bool f32_any_lane(bool x) {
+  return __builtin_amdgcn_readfirstlane(__syncthreads_or(x)) != 0;
+}
+
 // Row blocks of 32 per workgroup; SH wavefronts (2 or 4) share each.
 template <int D> constexpr int f32_fwd_blocks() { return D == 128 ? 4 : 2; }
 constexpr int kF32BwdBlocks = 2;
@@ -250,19 +271,26 @@ attn_fwd_f32(FwdArgs a) {
       for (int r = 0; r < 16; ++r) out[64 * (2 + 16 * mt + r)] = o[mt][r];
   }
   __syncthreads();
-  if (half > 0 || !qvalid) return;
+  if (half == 0) {
 #pragma unroll
-  for (int i = 0; i < SH - 1; ++i, part += PART) {
-    const float m1 = part[0], mm = fmaxf(m, m1);
-    const float w0 = m == -INFINITY ? 0.f : fast_exp2((m - mm) * kLog2e);
-    const float w1 = m1 == -INFINITY ? 0.f : fast_exp2((m1 - mm) * kLog2e);
-    m = mm;
-    l = l * w0 + part[64] * w1;
+    for (int i = 0; i < SH - 1; ++i, part += PART) {
+      const float m1 = part[0], mm = fmaxf(m, m1);
+      const float w0 = m == -INFINITY ? 0.f : fast_exp2((m - mm) * kLog2e);
+      const float w1 = m1 == -INFINITY ? 0.f : fast_exp2((m1 - mm) * kLog2e);
+      m = mm;
+      l = l * w0 + part[64] * w1;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) o[mt][r] = o[mt][r] * w0 + part[64 * (2 + 16 * mt + r)] * w1;
+        for (int r = 0; r < 16; ++r) o[mt][r] = o[mt][r] * w0 + part[64 * (2 + 16 * mt + r)] * w1;
+    }
   }
+  if ((a.causal || a.Tkv % 32 != 0) && f32_any_lane(half == 0 && qvalid && f32_any_nan(o))) {
+    for (int r = q0 + wave; r < min(q0 + BM, a.Tq); r += WAVES)
+      simt_fwd_row<float, D / 64>(a, D, (int64_t)bh * a.Tq + r);
+    return;
+  }
+  if (half > 0 || !qvalid) return;
   // no visible key: zeros; visible keys whose scores are all -inf: NaN, as exp(-inf + inf)
   const float inv = l > 0.f ? 1.0f / l : (n_kv > 0 ? __builtin_nanf("") : 0.f);
   f32_store_row<D>((float*)a.o + b * a.so_b + h * a.so_h + (int64_t)qrow * a.so_s, o, inv, g);
@@ -364,6 +392,11 @@ attn_bwd_dq_f32(BwdArgs a) {
     f32_cols<D>(of, Ks, s, dq);
   }
   f32_merge<MT, SH, PART>(reinterpret_cast<float*>(smem) + qb * 64 * 16 * MT + lane, dq, half);
+  if ((a.causal || a.Tkv % 32 != 0) && f32_any_lane(half == 0 && qvalid && f32_any_nan(dq))) {
+    for (int r = q0 + wave; r < min(q0 + BM, a.Tq); r += WAVES)
+      simt_dq_row<float, D / 64>(a, D, (int64_t)bh * a.Tq + r);  // reads the delta stored above
+    return;
+  }
   if (half == 0 && qvalid)
     f32_store_row<D>((float*)a.dq + b * a.sdq_b + h * a.sdq_h + (int64_t)qrow * a.sdq_s, dq, a.scale, g);
 }
@@ -456,6 +489,12 @@ attn_bwd_dkdv_f32(BwdArgs a) {
   float* part = reinterpret_cast<float*>(smem) + blk * 64 * 16 * MT + lane;
   f32_merge<MT, SH, PART>(part, dk, half);
   f32_merge<MT, SH, PART>(part, dv, half);
+  if ((a.causal || a.Tq % 32 != 0) &&
+      f32_any_lane(half == 0 && kvvalid && (f32_any_nan(dk) || f32_any_nan(dv)))) {
+    for (int r = kv0 + wave; r < min(kv0 + BN, a.Tkv); r += WAVES)
+      simt_dkdv_row<float, D / 64>(a, D, (int64_t)bhk * a.Tkv + r);
+    return;
+  }
   if (half == 0 && kvvalid) {
     f32_store_row<D>((float*)a.dk + b * a.sdk_b + hk * a.sdk_h + (int64_t)kvw * a.sdk_s, dk, a.scale, g);
     f32_store_row<D>((float*)a.dv + b * a.sdv_b + hk * a.sdv_h + (int64_t)kvw * a.sdv_s, dv, 1.f, g);

@@ -310,6 +310,55 @@ def test_attention_fp32_large_grid(causal):
                  grads=True)
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_attention_fp32_hidden_rows_that_are_not_finite(head_dim):
+    # keys and queries that the mask hides share 32-row blocks with visible ones and are
+    # multiplied by zero weights there: what they hold must not reach the result.  Rows
+    # that see no infinity or NaN equal the oracle on clean inputs
+    x = [randn((1, 2, 100, head_dim), torch.float32, 140 + i) for i in range(4)]  # q, k, v, do
+    eo, lse = oracle.attention.forward(*(np32(t) for t in x[:3]), True)
+    edq, edk, edv = oracle.attention.backward(np32(x[3]), *(np32(t) for t in x[:3]), lse, True)
+
+    def run(q, k, v, do):
+        q, k, v = (t.detach().requires_grad_(True) for t in (q, k, v))
+        o = tritium.attention(q, k, v)
+        o.backward(do)
+        return o, q.grad, k.grad, v.grad
+
+    # a cache longer than the queries, its unwritten rows NaN: no query sees them
+    k, v = (torch.cat([t, torch.full_like(t[:, :, :28], float("nan"))], 2) for t in x[1:3])
+    o, dq, dk, dv = run(x[0], k, v, x[3])
+    for got, want, name in ((o, eo, "o"), (dq, edq, "dq"), (dk[:, :, :100], edk, "dk"),
+                            (dv[:, :, :100], edv, "dv")):
+        assert_close(got, want, 1e-5, 1e-5, name)
+    assert not dk[:, :, 100:].any() and not dv[:, :, 100:].any()
+    # an infinite value and a NaN key: the rows before them
+    k, v = x[1].clone(), x[2].clone()
+    v[0, 0, 50, 3], k[0, 1, 52, 0] = float("inf"), float("nan")
+    o, dq, _, _ = run(x[0], k, v, x[3])
+    assert torch.isinf(o[0, 0, 50:, 3]).all() and torch.isnan(o[0, 1, 52:]).all()
+    assert_close(o[:, :, :50], eo[:, :, :50], 1e-5, 1e-5, "o")
+    assert_close(dq[:, :, :50], edq[:, :, :50], 1e-5, 1e-5, "dq")
+    # a NaN gradient and an infinite query: the keys after them
+    q, do = x[0].clone(), x[3].clone()
+    do[0, :, 20], q[0, :, 80] = float("nan"), float("inf")
+    _, _, dk, dv = run(q, x[1], x[2], do)
+    assert torch.isnan(dv[0, :, :21]).all() and torch.isnan(dk[0, :, :81]).any(-1).all()
+    assert_close(dk[:, :, 81:], edk[:, :, 81:], 1e-5, 1e-5, "dk")
+    assert_close(dv[:, :, 81:], edv[:, :, 81:], 1e-5, 1e-5, "dv")
+    do = x[3].clone()
+    do[0, :, 42, 1] = float("inf")
+    _, _, dk, dv = run(*x[:3], do)
+    assert torch.isinf(dv[0, :, :43, 1]).all()
+    assert_close(dk[:, :, 43:], edk[:, :, 43:], 1e-5, 1e-5, "dk")
+    assert_close(dv[:, :, 43:], edv[:, :, 43:], 1e-5, 1e-5, "dv")
+    # no mask, a last block that is not full: an infinite last value is an infinite output
+    v = x[2].clone()
+    v[0, 0, 99, 5] = float("inf")
+    o = tritium.attention(x[0], x[1], v, is_causal=False)
+    assert torch.isinf(o[0, 0, :, 5]).all() and torch.isfinite(o[0, 1]).all()
+
+
 def test_attention_fp32_unaligned_rows():
     x = [randn((1, 2, 70, 67), torch.float32, 71 + i)[..., 1:65] for i in range(3)]
     o = tritium.attention(*x)
