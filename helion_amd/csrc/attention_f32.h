@@ -42,7 +42,11 @@
 // weight of zero, and zero times an infinite or NaN element of the other
 // operand is NaN.  So a workgroup with masked pairs whose sums end in any NaN
 // takes its rows again with the SIMT code, which visits the visible pairs
-// only: what a hidden row holds never reaches the result.
+// only: what a hidden row holds never reaches the result.  The forward does so
+// for an infinite sum too: its weights reach 2^8 (lazy rescaling) where those
+// of the SIMT code reach 1, so values of 1e36 may overflow in its sums alone.
+// (A reference point that follows every row's maximum would do without, and
+// costs the forward another 2%.)
 
 // Per-lane byte offsets into a BTile of D fp32 (2 D 16-bit) columns: row
 // granule 2 i + g of row l32 (i < 8; a granule 16 columns of 16 bytes on is
@@ -160,6 +164,16 @@ struct F32Dma {
     else return (i >> 1) * 2 * P::BYTES + (i & 1) * 32 * P::RB;
   }
 };
+
+template <int MT>
+__device__ __forceinline__ bool f32_all_finite(const f32x16 (&v)[MT]) {
+  float z = 0.f;  // NaN once an infinity or a NaN has been multiplied by 0
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) z = fmaf(v[mt][r], 0.f, z);
+  return z == 0.f;
+}
 
 template <int MT>
 __device__ __forceinline__ bool f32_any_nan(const f32x16 (&v)[MT]) {
@@ -285,7 +299,7 @@ attn_fwd_f32(FwdArgs a) {
         for (int r = 0; r < 16; ++r) o[mt][r] = o[mt][r] * w0 + part[64 * (2 + 16 * mt + r)] * w1;
     }
   }
-  if ((a.causal || a.Tkv % 32 != 0) && f32_any_lane(half == 0 && qvalid && f32_any_nan(o))) {
+  if (f32_any_lane(half == 0 && qvalid && !f32_all_finite(o))) {
     for (int r = q0 + wave; r < min(q0 + BM, a.Tq); r += WAVES)
       simt_fwd_row<float, D / 64>(a, D, (int64_t)bh * a.Tq + r);
     return;

@@ -359,6 +359,21 @@ def test_attention_fp32_hidden_rows_that_are_not_finite(head_dim):
     assert torch.isinf(o[0, 0, :, 5]).all() and torch.isfinite(o[0, 1]).all()
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_attention_fp32_values_near_the_largest(head_dim):
+    # key 130 scores 5.4 above the keys before it: a weight of e^5.4 = 221 would take a
+    # value of 2e36 past the largest float32, 3.4e38, which the running sum itself stays
+    # below (at most 160 weights of 1, 3.2e38).  Every value is the same, so the output is
+    # that value, within the roundings of a sum of 160 terms
+    q = torch.zeros((1, 1, 64, head_dim), device="cuda")
+    k = torch.zeros((1, 1, 160, head_dim), device="cuda")
+    q[..., 0] = 1.0
+    k[:, :, 130, 0] = 5.4 * head_dim ** 0.5
+    v = torch.full((1, 1, 160, head_dim), 2e36, device="cuda")
+    o = tritium.attention(q, k, v, is_causal=False)
+    assert_close(o / 2e36, np.ones(o.shape), 160 * 2.0 ** -24, 0.0)
+
+
 def test_attention_fp32_unaligned_rows():
     x = [randn((1, 2, 70, 67), torch.float32, 71 + i)[..., 1:65] for i in range(3)]
     o = tritium.attention(*x)
