@@ -2766,18 +2766,22 @@ attn_decode_kernel(DecArgs a) {
 // end.  Register r of S^T block u
 // holds key 16 u + 4 g + r (g = lane >> 4), which is the operand order of the
 // P^T that follows; V^T comes from transposing LDS reads of the same keys.
-// P enters the product as a sum of three 16-bit terms, which hold all 24 bits
-// of the fp32 weight.  (For fp16, whose terms would lose bits below 2^-24,
-// weights are formed 2^7 larger; the reference point of the partials accounts
-// for it.)  A non-finite key or value turns such a sum into NaN where the
-// plain product may be infinite, so a chunk that ends in any NaN is done
-// again by dec_chunk.
+// The weights stay fp32: for bf16, P enters the product as a sum of three
+// bf16 terms, which hold all 24 bits; three fp16 terms would not (a weight
+// below 2^-9 would lose bits to their exponent range), so for fp16 the product
+// runs on the fp32 matrix instruction, V widened on the way (eight 16 x 16 x 4
+// in place of three 16 x 16 x 32: 50.6 us against 46.5 at [8, 32, 8, 8192,
+// 128]).  A non-finite key or value may turn either sum into NaN where the
+// plain product is infinite (the lower terms' signs; a key past the chunk's
+// end, whose weight is 0), so a chunk that ends in any NaN is done again by
+// dec_chunk.
 //
-// Bound: HBM.  Graph replays, same box, dec_chunk's kernel -> this one:
+// Bound: HBM.  Graph replays, same box, dec_chunk's kernel -> this one, bf16:
 // [8, 32, 8, 8192, 128] 54.0 -> 47.0 us (5.7 TB/s with the combine), [32, 32,
 // 8, 2048, 128] 53.2 -> 47.8, [1, 32, 8, 4096, 128] 18.2 -> 11.6, [10, 12, 3,
 // 9149, 64] 25.1 -> 21.9, [3, 32, 4, 16000, 64] 33.0 -> 17.4, [1, 16, 2,
-// 2000, 64] 18.9 -> 7.5; with groups of one and two heads it is equal or up
+// 2000, 64] 18.9 -> 7.5; fp16: the first three 57.5 -> 50.6, 56.8 -> 50.2,
+// 17.4 -> 13.4, [10, 12, 3, 9149, 64] 25.4 -> 25.1; with groups of one and two heads it is equal or up
 // to 4% slower, so those stay on the kernel above.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 template <typename T>
@@ -2810,7 +2814,7 @@ attn_decode_mfma(DecArgs a) {
   constexpr int TILE = 32 * P::RB, RING = kDecRing, STAGES = RING / (2 * TILE);
   constexpr int DMAS = TILE / 1024;          // per 32-row tile
   constexpr int NV = D == 128 ? 4 : 2;       // DMAs after which the swizzle repeats
-  constexpr float SHIFT = std::is_same<T, f16_t>::value ? 7.f : 0.f;
+  constexpr bool TERMS = std::is_same<T, bf16_t>::value;  // P as three 16-bit terms
   static_assert(STAGES >= 1 && dec_lds_floats(W, GMAX, D) * 4 <= W * RING, "LDS");
   __shared__ __attribute__((aligned(1024))) char smem[W * RING];
   const int lane = threadIdx.x & 63, wave = wave_id();
@@ -2866,7 +2870,7 @@ attn_decode_mfma(DecArgs a) {
   f32x4 o[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) o[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, nm = SHIFT, l = 0.f;
+  float m = -INFINITY, nm = 0.f, l = 0.f;
 #pragma unroll
   for (int t = 0; t < STAGES; ++t)
     if (t < n) issue(t);
@@ -2900,7 +2904,7 @@ attn_decode_mfma(DecArgs a) {
       const float m_new = fmaxf(m, mx);
       const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);
       m = m_new;
-      nm = m == -INFINITY ? SHIFT : SHIFT - m;
+      nm = m == -INFINITY ? 0.f : -m;
       l *= alpha;
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) o[mt] *= alpha;
@@ -2912,10 +2916,14 @@ attn_decode_mfma(DecArgs a) {
       for (int r = 0; r < 4; ++r) {
         float x = fast_exp2(fmaf(s[u][r], a.sl2, nm));
         l += x;
+        if constexpr (TERMS) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          p[k][4 * u + r] = (T)x;
-          x -= (float)p[k][4 * u + r];
+          for (int k = 0; k < 3; ++k) {
+            p[k][4 * u + r] = (T)x;
+            x -= (float)p[k][4 * u + r];
+          }
+        } else {
+          s[u][r] = x;
         }
       }
     // V^T operands: in each 16-lane group, lane s addresses row 4 g + (s >> 2)
@@ -2929,8 +2937,14 @@ attn_decode_mfma(DecArgs a) {
       const v4s hi =
           __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(lds_addr(Vs + P::off(16 + r0, c) + sub)));
       const V v = __builtin_bit_cast(V, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      if constexpr (TERMS) {
 #pragma unroll
-      for (int k = 0; k < 3; ++k) o[mt] = mma16<T>(v, p[k], o[mt]);
+        for (int k = 0; k < 3; ++k) o[mt] = mma16<T>(v, p[k], o[mt]);
+      } else {  // register (u, r) holds the keys 16 u + 4 g + r of both operands
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          o[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)v[i], s[i >> 2][i & 3], o[mt], 0, 0, 0);
+      }
     }
     // every LDS read of this stage has returned before its DMA is reissued
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -2952,7 +2966,7 @@ attn_decode_mfma(DecArgs a) {
   }
   if (l16 < group) {
     if (g == 0) {
-      sm[wave * GMAX + l16] = m == -INFINITY ? m : m - SHIFT;
+      sm[wave * GMAX + l16] = m;
       sl[wave * GMAX + l16] = l;
     }
 #pragma unroll

@@ -399,6 +399,27 @@ def test_attention_decode_routes(dtype, head_dim, b, h, hkv, kv_len):
     assert_close(lse, e_lse, 1e-4, 1e-4, "lse")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("e", [12, 20, 30, 36])
+def test_attention_decode_small_weights(dtype, head_dim, e):
+    # key 0 takes almost the whole weight and its value is zero: the output is made of
+    # weights near 2^-e alone, which keep their fp32 precision in the groups' matrix kernel.
+    # Bound: the rounding to 16 bits (2^-8 or 2^-11 of the value, 2^-25 where fp16 is
+    # subnormal), and 2^-17 for the exponent of a weight formed in fp32 (scores up to 64)
+    q, k = torch.zeros((1, 8, 1, head_dim)), torch.zeros((1, 2, 512, head_dim))
+    q[..., 0], k[:, :, 0, 0] = 8.0, e * float(np.log(2.0)) * head_dim ** 0.5 / 8.0
+    q[..., 1:9] = randn((1, 8, 1, 8), seed=93, device="cpu")
+    k[:, :, 1:, 1:9] = randn((1, 2, 511, 8), seed=94, device="cpu", scale=0.3)
+    v = randn((1, 2, 512, head_dim), seed=95, device="cpu").abs() * 40 * 2.0 ** min(e, 8)
+    v[:, :, 0] = 0
+    q, k, v = (t.to(dtype).cuda() for t in (q, k, v))
+    o = tritium.attention(q, k, v, is_causal=False)
+    eo, _ = oracle.attention.forward(np32(q), np32(k), np32(v), False)
+    half_ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert_close(o, eo, half_ulp + 2.0 ** -17, 2.0 ** -25 if dtype == torch.float16 else 0.0)
+
+
 def test_attention_decode_infinite_value():
     # an infinite value is an infinite output in its column, not a NaN (the split weights'
     # lower terms multiply it by zero or by a negative number)
