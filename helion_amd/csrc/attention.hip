@@ -2611,6 +2611,12 @@ __device__ __forceinline__ void dec_merge(float& m, float& l, float (&o)[N], flo
   m = mx;
 }
 
+// lse of a head (m in log2 units): NaN where every score is -inf, whether the
+// weights' sum came out as NaN (exp(-inf + inf)) or as 0.
+__device__ __forceinline__ float dec_lse(float m, float l) {
+  return l > 0.f ? (m + log2f(l)) * kLn2 : __builtin_nanf("");
+}
+
 // LDS of a workgroup of `waves` wavefronts: per wavefront and head m, l, o[D].
 constexpr int dec_lds_floats(int waves, int heads, int D) { return waves * heads * (D + 2); }
 
@@ -2634,7 +2640,7 @@ __device__ __forceinline__ void dec_write(const DecArgs& a, const float* sm, int
     const int hq = hk * group + g;
     if (a.n_splits == 1) {
       ((T*)a.o + b * a.so_b + hq * a.so_h)[d] = from_f32<T>(ll > 0.f ? oo[0] / ll : 0.f);
-      if (d == 0) a.lse[(int64_t)b * a.H + hq] = (mm + log2f(ll)) * kLn2;
+      if (d == 0) a.lse[(int64_t)b * a.H + hq] = dec_lse(mm, ll);
     } else {
       float* dst = a.part + (((int64_t)b * a.H + hq) * a.n_splits + split) * (D + 2);
       dst[2 + d] = oo[0];
@@ -3017,7 +3023,7 @@ attn_decode_combine(DecArgs a) {
   for (int c = 0; c < a.n_splits; ++c) od += src[c * (D + 2) + 2 + threadIdx.x] * wgt[c];
   T* orow = (T*)a.o + b * a.so_b + h * a.so_h;
   orow[threadIdx.x] = from_f32<T>(l > 0.f ? od / l : 0.f);
-  if (threadIdx.x == 0) a.lse[bh] = (mx + log2f(l)) * kLn2;
+  if (threadIdx.x == 0) a.lse[bh] = dec_lse(mx, l);
 }
 
 // --------------------------------------------------------------- SIMT path --

@@ -420,6 +420,20 @@ def test_attention_decode_small_weights(dtype, head_dim, e):
     assert_close(o, eo, half_ulp + 2.0 ** -17, 2.0 ** -25 if dtype == torch.float16 else 0.0)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kv_len", [200, 517, 5000])
+def test_attention_decode_every_score_minus_infinity(dtype, kv_len):
+    # the same answer whatever the heads per kv head (vector and matrix kernels, one chunk
+    # and several): an lse of NaN, an output of zero
+    from helion_amd.attention import _attention_forward
+    for hkv in (4, 2, 1):
+        q = torch.ones((1, 4, 1, 64), dtype=dtype, device="cuda")
+        k, v = (randn((1, hkv, kv_len, 64), dtype, 96 + i) for i in range(2))
+        k[..., 0] = float("-inf")
+        o, lse = _attention_forward(q, k, v, False)
+        assert torch.isnan(lse).all() and not o.any(), hkv
+
+
 def test_attention_decode_infinite_value():
     # an infinite value is an infinite output in its column, not a NaN (the split weights'
     # lower terms multiply it by zero or by a negative number)
