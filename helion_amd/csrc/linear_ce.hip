@@ -592,15 +592,16 @@ double split_cost(int64_t tiles, int64_t k_tiles, int64_t s) {
   return rounds * (1.8 * (double)cdiv(k_tiles, s) + 5.0) + partials;
 }
 
-// K splits of `tiles` output tiles (at most 16, at least 16 K tiles each):
-// the cheapest by split_cost.  A power of two that filled the GPU twice left
-// 384 workgroups on 256 compute units for the 48 tiles of dH at 4091 x 768
-// (50257 rows reduced): 8 splits 429 us with their sum, 5 splits 342.
+// K splits of `tiles` output tiles (at most 16, at least 16 K tiles each, at
+// most max_parts tiles of fp32 partials): the cheapest by split_cost.  A power
+// of two that filled the GPU twice left 384 workgroups on 256 compute units
+// for the 48 tiles of dH at 4091 x 768 (50257 rows reduced): 8 splits 429 us
+// with their sum, 5 splits 342.
 template <typename T>
-int split_count(int64_t tiles, int64_t K) {
+int split_count(int64_t tiles, int64_t K, int64_t max_parts) {
   const int64_t kt = cdiv(K, gemm::bk<CfgT<T>, T>());
   int64_t best = 1;
-  for (int64_t s = 2; s <= 16 && kt / s >= 16; ++s)
+  for (int64_t s = 2; s <= 16 && kt / s >= 16 && s * tiles <= max_parts; ++s)
     if (even_splits(kt, s) == s && split_cost<T>(tiles, kt, s) < split_cost<T>(tiles, kt, best))
       best = s;
   return (int)best;
@@ -609,9 +610,13 @@ int split_count(int64_t tiles, int64_t K) {
 // An M x N product over K as `body` rows (whole rounds of tiles, one pass)
 // and the other rows cut into `splits` K ranges: 591 tiles are 2.3 rounds of
 // 256 compute units, and a third round that is a third full costs as much as
-// a full one (dW [50257, 768] over 4091 tokens 369 -> 332 us).
+// a full one (dW [50257, 768] over 4091 tokens 369 -> 332 us).  The partials
+// stay small beside the chunk's G: those of a rest fill at most one round
+// (64 MiB for 256 tiles of 256 x 256), and a product split as a whole has
+// fewer than four rounds of them, so grids of two rounds and more are never
+// split as a whole.
 struct RowPlan {
-  int64_t body;
+  int64_t body;  // M: no split
   int splits;
 };
 template <typename T>
@@ -619,12 +624,17 @@ RowPlan row_plan(int64_t M, int64_t N, int64_t K) {
   typedef CfgT<T> C;
   const int64_t kt = cdiv(K, gemm::bk<C, T>());
   const int64_t tm = cdiv(M, C::BM), tn = cdiv(N, C::BN), cus = cu_count();
-  RowPlan best{0, split_count<T>(tm * tn, K)};
-  double cost = split_cost<T>(tm * tn, kt, best.splits);
+  RowPlan best{M, 1};
+  double cost = split_cost<T>(tm * tn, kt, 1);
+  const int all = split_count<T>(tm * tn, K, 4 * cus - 1);
+  if (all > 1) {
+    best = RowPlan{0, all};
+    cost = split_cost<T>(tm * tn, kt, all);
+  }
   const int64_t rounds = tm * tn / cus, body = rounds * cus / tn;
   if (rounds > 0 && body > 0 && body < tm) {
     const int64_t rest = (tm - body) * tn;
-    const int s = split_count<T>(rest, K);
+    const int s = split_count<T>(rest, K, cus);
     const double c = split_cost<T>(body * tn, kt, 1) + split_cost<T>(rest, kt, s) + 5.0;
     if (s > 1 && c < cost) best = RowPlan{body * C::BM, s};
   }
@@ -633,15 +643,16 @@ RowPlan row_plan(int64_t M, int64_t N, int64_t K) {
 
 struct BwdLayout {
   int64_t chunk, n_chunks, ld_g;
-  int sh;  // K splits of dH
-  size_t n_valid, gm, dh_acc, dw_part, total;
+  RowPlan dh;  // dH's token rows
+  size_t n_valid, gm, dh_acc, dh_part, dw_part, total;
 };
 
 // The backward's workspace: the count of valid rows, G of one vocabulary
 // chunk [N, ld_g] (chunk rows chosen so that G fits kGBudget bytes, or
-// chunk_rows rounded up to the row tile), the fp32 dH accumulator [sh, N, D]
-// when there is more than one chunk or dH is split over K, and the fp32
-// partials of the dW rows that are split over tokens.
+// chunk_rows rounded up to the row tile), the fp32 accumulator of dH's rows
+// that are not split when there is more than one chunk, the fp32 partials of
+// those that are split over the vocabulary, and the fp32 partials of the dW
+// rows that are split over tokens.
 template <typename T>
 BwdLayout bwd_layout(int64_t N, int64_t D, int64_t V, bool need_dh, bool need_dw,
                      int64_t chunk_rows) {
@@ -662,17 +673,17 @@ BwdLayout bwd_layout(int64_t N, int64_t D, int64_t V, bool need_dh, bool need_dw
     off += (size_t)round_up((int64_t)bytes, 256);
     return at;
   };
-  L.sh = need_dh ? split_count<T>(cdiv(N, CfgT<T>::BM) * cdiv(D, CfgT<T>::BN), std::min(chunk, V)) : 1;
+  L.dh = need_dh ? row_plan<T>(N, D, std::min(chunk, V)) : RowPlan{N, 1};
   // fp32 partials of dW's split rows, over the whole chunks and the last one
   size_t dw_bytes = 0;
   for (const int64_t vc : {std::min(chunk, V), V - (L.n_chunks - 1) * chunk}) {
     const RowPlan p = row_plan<T>(vc, D, N);
-    if (need_dw && p.splits > 1)
-      dw_bytes = std::max(dw_bytes, (size_t)p.splits * (size_t)(vc - p.body) * D * 4);
+    if (need_dw) dw_bytes = std::max(dw_bytes, (size_t)p.splits * (size_t)(vc - p.body) * D * 4);
   }
   L.n_valid = take(4);
   L.gm = take((size_t)N * L.ld_g * esz);
-  L.dh_acc = (need_dh && (L.n_chunks > 1 || L.sh > 1)) ? take((size_t)L.sh * N * D * 4) : 0;
+  L.dh_acc = (need_dh && L.n_chunks > 1) ? take((size_t)L.dh.body * D * 4) : 0;
+  L.dh_part = take((size_t)L.dh.splits * (size_t)(N - L.dh.body) * D * 4);
   L.dw_part = dw_bytes > 0 ? take(dw_bytes) : 0;
   L.total = off;
   return L;
@@ -762,7 +773,8 @@ int bwd_impl(const float* grad_out, const void* hidden, const void* weight, cons
   lce_count_valid<TT><<<1, 1024, 0, st>>>((const TT*)target, N, ignore_index, n_valid);
   if (int e = check_launch("linear_ce count")) return e;
   T* gm = (T*)(w + L.gm);
-  float* dh_acc = L.dh_acc ? (float*)(w + L.dh_acc) : nullptr;
+  float* dh_acc = (float*)(w + L.dh_acc);
+  float* dh_part = (float*)(w + L.dh_part);
   float* dw_part = L.dw_part ? (float*)(w + L.dw_part) : nullptr;
   for (int64_t c = 0; c < L.n_chunks; ++c) {
     const int64_t vc0 = c * L.chunk;
@@ -787,7 +799,7 @@ int bwd_impl(const float* grad_out, const void* hidden, const void* weight, cons
       // both MN-contiguous; each row's token reduction in one product, or in
       // fp32 partials summed in order, rounded once
       const RowPlan plan = row_plan<T>(vc, D, N);
-      const int64_t whole = plan.splits > 1 ? plan.body : vc, rest = vc - whole;
+      const int64_t whole = plan.body, rest = vc - whole;
       T* dst = (T*)dweight + vc0 * D;
       if (whole > 0) {
         gemm::Problem p{gm, hidden, L.ld_g, D, whole, D, N};
@@ -802,21 +814,28 @@ int bwd_impl(const float* grad_out, const void* hidden, const void* weight, cons
       }
     }
     if (need_dh) {
-      // dH[N, D] (+)= G W_c: A = G (K-contiguous), B[d][v] = W_c[v][d] (MN-contiguous);
-      // with one chunk and no split straight into dH, else into sh fp32
-      // accumulators (one per K split, each summed over the chunks in order)
-      // that a fixed-order sum rounds once after the last chunk
-      gemm::Problem p{gm, wc, L.ld_g, D, N, D, vc};
+      // dH[N, D] (+)= G W_c: A = G (K-contiguous), B[d][v] = W_c[v][d] (MN-contiguous).
+      // Rows in one pass: straight into dH with one chunk, else summed over the
+      // chunks in fp32 and rounded with the last.  Rows split over the chunk's
+      // vocabulary: fp32 partials (one per range, each summed over the chunks in
+      // order) that a fixed-order sum rounds once after the last chunk.
       const bool last = c + 1 == L.n_chunks;
-      if (dh_acc == nullptr) {
-        if (int e = gemm_store<T, false, true>(p, nullptr, dhidden, false, D, st)) return e;
-      } else if (L.sh == 1 && last) {
-        if (int e = gemm_store<T, false, true>(p, dh_acc, dhidden, false, D, st)) return e;
-      } else {
-        if (int e = gemm_store<T, false, true>(p, c > 0 ? dh_acc : nullptr, dh_acc, true, D, st, L.sh))
+      const int64_t whole = L.dh.body, rest = N - whole;
+      if (whole > 0) {
+        gemm::Problem p{gm, wc, L.ld_g, D, whole, D, vc};
+        const float* in = c > 0 ? dh_acc : nullptr;
+        if (int e = last ? gemm_store<T, false, true>(p, in, dhidden, false, D, st)
+                         : gemm_store<T, false, true>(p, in, dh_acc, true, D, st))
+          return e;
+      }
+      if (rest > 0) {
+        gemm::Problem p{gm + whole * L.ld_g, wc, L.ld_g, D, rest, D, vc};
+        if (int e = gemm_store<T, false, true>(p, c > 0 ? dh_part : nullptr, dh_part, true, D, st,
+                                               L.dh.splits))
           return e;
         if (last) {
-          if (int e = tritium_sum_splits(dh_acc, dhidden, L.sh, N * D, std::is_same<T, bf16_t>::value ? kBF16 : kF16, st))
+          if (int e = tritium_sum_splits(dh_part, (T*)dhidden + whole * D, L.dh.splits, rest * D,
+                                         std::is_same<T, bf16_t>::value ? kBF16 : kF16, st))
             return e;
         }
       }

@@ -67,3 +67,17 @@ def test_attention_bwd_workspace_size_and_rejection():
     assert rc == 1
     assert b"dS workspace" in handle.tritium_last_error()
 
+
+@pytest.mark.skipif(not os.path.exists(L.LIB_PATH), reason="library not built")
+@pytest.mark.parametrize("n,d,v,partials", [
+    (8192, 4096, 128256, 128), (8320, 4096, 128256, 128), (8576, 4096, 128256, 128),
+    (10624, 8192, 50257, 128), (4091, 768, 50257, 320), (4160, 4096, 128256, 320),
+    (4608, 4096, 128256, 320), (128, 768, 50257, 320)])
+def test_linear_ce_bwd_workspace_is_bounded(n, d, v, partials):
+    # G of one vocabulary chunk (at most 1 GiB), an fp32 dH when there are several, and the
+    # partials of split products: a rest of one round of 256 tiles of 256 x 256 (64 MiB) in
+    # each product, or below four rounds (256 MiB) of dH where its grid is less than two
+    size = L.lib().tritium_linear_ce_bwd_workspace_size(n, d, v, 2, 1, 1, 0)
+    chunk = min(v, 2 ** 30 // (2 * n) // 256 * 256)
+    fixed = 2 * n * (chunk + 7) + (4 * n * d if chunk < v else 0) + 4096
+    assert 2 * n * chunk <= size <= fixed + partials * 2 ** 20

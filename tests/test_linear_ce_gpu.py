@@ -200,6 +200,47 @@ def test_linear_ce_mfma_backward_edges(dtype, n, d, v, ignore_frac, tdtype, chun
     _run(n, d, v, dtype, seed=20, ignore_frac=ignore_frac, tdtype=tdtype, chunk_rows=chunk)
 
 
+def _row_errors(got, want):
+    """Relative error of every row (2-norm over the row's, at least the mean row's)."""
+    norm = want.norm(dim=1)
+    return (got.float() - want).norm(dim=1) / norm.clamp(min=float(norm.mean()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,d,v,chunk", [
+    (2100, 768, 50257, 0),      # dW: 591 tiles, 512 in two rounds and ragged rows over 2 token ranges
+    (8300, 2048, 20001, 0),     # dW and dH (264 tiles, 8 of them over the vocabulary)
+    (8300, 2048, 20001, 16384), # the same, dH summed over two chunks of unlike length
+])
+def test_linear_ce_backward_whole_rounds_and_split_rest(dtype, n, d, v, chunk):
+    # grids with a badly filled last round: the rows of whole rounds in one product, the
+    # others split over the reduction; every row against fp32 products.  G and the result
+    # are rounded to 16 bits (2^-8 of a value at most, in bf16): 2^-8 for each, and as much
+    # for the sums.  The loss is scaled by 2^14, as training in fp16 does: the entries of G
+    # (1 / (v n) = 1e-8 here) would be subnormal in fp16
+    print(f"[lce bwd] {dtype} n={n} d={d} v={v} chunk={chunk}", flush=True)
+    h, w, t = _inputs(n, d, v, dtype, seed=30, ignore_frac=0.01)
+    _, lse = tritium.linear_ce._linear_cross_entropy_forward(h, w, t)
+    dh, dw = tritium.linear_ce._backward(torch.tensor(2.0 ** 14, device="cuda"), h, w, t, lse,
+                                         True, True, -100, chunk)
+    hf, wf = h.float(), w.float()
+    keep = t != -100
+    g = torch.softmax(hf @ wf.t(), 1)
+    g[keep.nonzero()[:, 0], t[keep]] -= 1.0
+    g *= (2.0 ** 14 * keep / keep.sum())[:, None]
+    for got, want, name in ((dw, g.t() @ hf, "dweight"), (dh, g @ wf, "dhidden")):
+        err = _row_errors(got, want)
+        assert float(err.max()) < 3 * 2.0 ** -8, f"{name} row {int(err.argmax())}: {float(err.max()):.3e}"
+
+
+@pytest.mark.parametrize("n,d,v,chunk", [
+    (300, 64, 6200, 3072),   # dH over 3 ranges; the last chunk (56 rows) fills one of them
+    (300, 64, 10400, 5120),  # 5 ranges; the last chunk (160 rows) three
+])
+def test_linear_ce_backward_last_chunk_with_fewer_ranges(n, d, v, chunk):
+    _run(n, d, v, torch.bfloat16, seed=31, ignore_frac=0.02, chunk_rows=chunk)
+
+
 def test_linear_ce_confident_targets():
     # targets at each row's arg-max with large logits: p(target) is close to 1 and the
     # target entry of G is a small difference p - 1
