@@ -641,6 +641,21 @@ RowPlan row_plan(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
+// The plan of dW's rows [vc0, vc0 + chunk) of V, relative to vc0.  A chunk of
+// two rounds of tiles and more takes its part of the plan for all V rows, so a
+// row's sum over the tokens does not depend on how the vocabulary was cut; a
+// smaller one, whose grid alone would leave the GPU idle, is planned by itself.
+template <typename T>
+RowPlan dw_plan(int64_t N, int64_t D, int64_t V, int64_t chunk, int64_t vc0) {
+  typedef CfgT<T> C;
+  const int64_t vc = std::min(chunk, V - vc0);
+  if (cdiv(std::min(chunk, V), C::BM) * cdiv(D, C::BN) < 2 * (int64_t)cu_count())
+    return row_plan<T>(vc, D, N);
+  RowPlan p = row_plan<T>(V, D, N);
+  p.body = std::max<int64_t>(0, std::min(vc, p.body - vc0));
+  return p;
+}
+
 struct BwdLayout {
   int64_t chunk, n_chunks, ld_g;
   RowPlan dh;  // dH's token rows
@@ -674,11 +689,11 @@ BwdLayout bwd_layout(int64_t N, int64_t D, int64_t V, bool need_dh, bool need_dw
     return at;
   };
   L.dh = need_dh ? row_plan<T>(N, D, std::min(chunk, V)) : RowPlan{N, 1};
-  // fp32 partials of dW's split rows, over the whole chunks and the last one
+  // fp32 partials of dW's split rows, the most of any chunk
   size_t dw_bytes = 0;
-  for (const int64_t vc : {std::min(chunk, V), V - (L.n_chunks - 1) * chunk}) {
-    const RowPlan p = row_plan<T>(vc, D, N);
-    if (need_dw) dw_bytes = std::max(dw_bytes, (size_t)p.splits * (size_t)(vc - p.body) * D * 4);
+  for (int64_t vc0 = 0; need_dw && vc0 < V; vc0 += chunk) {
+    const RowPlan p = dw_plan<T>(N, D, V, chunk, vc0);
+    dw_bytes = std::max(dw_bytes, (size_t)p.splits * (size_t)(std::min(chunk, V - vc0) - p.body) * D * 4);
   }
   L.n_valid = take(4);
   L.gm = take((size_t)N * L.ld_g * esz);
@@ -798,7 +813,7 @@ int bwd_impl(const float* grad_out, const void* hidden, const void* weight, cons
       // dW[vc0 : vc0 + vc, :] = G^T H: A[v][n] = G[n][v] and B[d][n] = H[n][d],
       // both MN-contiguous; each row's token reduction in one product, or in
       // fp32 partials summed in order, rounded once
-      const RowPlan plan = row_plan<T>(vc, D, N);
+      const RowPlan plan = dw_plan<T>(N, D, V, L.chunk, vc0);
       const int64_t whole = plan.body, rest = vc - whole;
       T* dst = (T*)dweight + vc0 * D;
       if (whole > 0) {

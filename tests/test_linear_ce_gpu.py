@@ -260,8 +260,9 @@ def test_linear_ce_confident_targets():
 
 
 def test_linear_ce_chunking_only_changes_dhidden_rounding():
-    # one chunk vs four: dweight's rows are the same products (bitwise), dhidden
-    # differs only by the fp32 accumulation across chunks before its one rounding
+    # one chunk vs four: dweight's rows are the same products (bitwise; 512 tokens are never
+    # split, the test below is of more), dhidden differs only by the fp32 accumulation
+    # across chunks before its one rounding
     h, w, t = _inputs(512, 256, 1024, torch.bfloat16, seed=22, ignore_frac=0.03)
     loss, lse = tritium.linear_ce._linear_cross_entropy_forward(h, w, t)
     g = torch.tensor(0.75, device="cuda")
@@ -270,6 +271,21 @@ def test_linear_ce_chunking_only_changes_dhidden_rounding():
     assert torch.equal(dw1, dw4)
     x, y = dh4.double(), dh1.double()
     assert float((x - y).norm() / y.norm()) < 5e-3
+
+
+def test_linear_ce_chunking_does_not_change_split_dweight_rows():
+    # tokens enough to split (8300), chunks of two rounds of tiles and more: rows past the
+    # whole rounds of the vocabulary's tiles are split over the tokens, the same rows in the
+    # same ranges however the vocabulary is cut (one chunk; two with the boundary inside the
+    # split rows or at their start)
+    h, w, t = _inputs(8300, 2048, 20001, torch.bfloat16, seed=32, ignore_frac=0.03)
+    _, lse = tritium.linear_ce._linear_cross_entropy_forward(h, w, t)
+    g = torch.tensor(0.75, device="cuda")
+    dh1, dw1 = tritium.linear_ce._backward(g, h, w, t, lse, True, True, -100, 0)
+    for chunk in (18432, 17408, 16384):
+        dh, dw = tritium.linear_ce._backward(g, h, w, t, lse, True, True, -100, chunk)
+        assert torch.equal(dw, dw1), chunk
+        assert float((dh.double() - dh1.double()).norm() / dh1.double().norm()) < 5e-3, chunk
 
 
 def test_linear_ce_autograd_keeps_no_logit_buffer_and_retain_graph():
