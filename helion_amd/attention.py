@@ -1,6 +1,6 @@
 """``attention`` on gfx950 HIP kernels (bf16/fp16 MFMA for head_dim 16-256,
-fp32 MFMA for head_dim 64 and 128; other fp32 head_dims, unaligned rows, and
-16-bit head_dims 512 and 1024, on a SIMT path).
+fp32 MFMA for head_dim 64 and 128; other fp32 head_dims, unaligned rows, rows
+that see only a few others, and 16-bit head_dims 512 and 1024, on a SIMT path).
 
 Drop-in for alkinun/helion ``tritium/ops/attention.py``: same signature
 (``attention(q, k, v, *, is_causal=True)`` 739-757), validation and messages

@@ -31,9 +31,9 @@
 //            no second S and dP, at the price of the dS traffic.
 //
 // fp32 inputs with head_dim 64 or 128 and 16-byte aligned rows run the fp32
-// matrix kernels of attention_f32.h; the other fp32 calls (and 16-bit ones
-// with head_dim outside the MFMA set, up to 1024) a SIMT path: one wavefront
-// per row, exact fp32 arithmetic.
+// matrix kernels of attention_f32.h, unless their rows see only a few others;
+// the other fp32 calls (and 16-bit ones with head_dim outside the MFMA set, up
+// to 1024) a SIMT path: one wavefront per row, exact fp32 arithmetic.
 //
 // Workgroup order is XCD-aware: the 8 XCDs receive workgroups round-robin, so
 // block ids are remapped to give every XCD a contiguous range of

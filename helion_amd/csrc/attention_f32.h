@@ -229,7 +229,7 @@ attn_fwd_f32(FwdArgs a) {
   for (int mt = 0; mt < MT; ++mt) o[mt] = zero16();
   float m = -INFINITY, nm = 0.f, l = 0.f;  // nm: -m, 0 while m is -inf
 
-  const int kv_end = a.causal ? min(a.Tkv, q0 + BM) : a.Tkv;
+  const int kv_end = a.causal ? min(a.Tkv, min(q0 + BM, a.Tq)) : a.Tkv;
   const int n_kv = (int)cdiv(kv_end, BK);
   F32Dma<D, WAVES> dma;
   dma.init(a.sk_s, a.sv_s);
@@ -240,7 +240,7 @@ attn_fwd_f32(FwdArgs a) {
     if (it + 1 < n_kv)
       dma.template issue<SH / 2>(smem + ((it + 1) & 1) * STAGE, kp, a.sk_s, vp, a.sv_s, BK * (it + 1), a.Tkv);
     const int kb = BK * it + 32 * half;  // this wavefront's 32 keys
-    if (kb >= a.Tkv || (a.causal && kb > qw0 + 31)) continue;
+    if (qw0 >= a.Tq || kb >= a.Tkv || (a.causal && kb > qw0 + 31)) continue;
     const char* Ks = smem + (it & 1) * STAGE + F32Dma<D, WAVES>::template rows_at<SH>(half);
     const char* Vs = Ks + P::BYTES;
     f32x16 s = f32_rows<D>(of, Ks, qf, zero16());
@@ -382,7 +382,7 @@ attn_bwd_dq_f32(BwdArgs a) {
   f32x16 dq[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) dq[mt] = zero16();
-  const int kv_end = a.causal ? min(a.Tkv, q0 + BM) : a.Tkv;
+  const int kv_end = a.causal ? min(a.Tkv, min(q0 + BM, a.Tq)) : a.Tkv;
   const int n_kv = (int)cdiv(kv_end, BK);
   F32Dma<D, WAVES> dma;
   dma.init(a.sk_s, a.sv_s);
@@ -393,7 +393,7 @@ attn_bwd_dq_f32(BwdArgs a) {
     if (it + 1 < n_kv)
       dma.template issue<SH / 2>(smem + ((it + 1) & 1) * STAGE, kp, a.sk_s, vp, a.sv_s, BK * (it + 1), a.Tkv);
     const int kb = BK * it + 32 * half;
-    if (kb >= a.Tkv || (a.causal && kb > qw0 + 31)) continue;
+    if (qw0 >= a.Tq || kb >= a.Tkv || (a.causal && kb > qw0 + 31)) continue;
     const char* Ks = smem + (it & 1) * STAGE + F32Dma<D, WAVES>::template rows_at<SH>(half);
     const char* Vs = Ks + P::BYTES;
     f32x16 s = f32_rows<D>(of, Ks, qf, zero16());
@@ -439,18 +439,27 @@ attn_bwd_dkdv_f32(BwdArgs a) {
   const int kv0 = kt * BN, kvb = kv0 + 32 * blk, kvw = kvb + l32;
   const bool kvvalid = kvw < a.Tkv;
 
+  const int q_begin = a.causal ? kv0 : 0;  // top-left causal: rows < kv0 see none
+  const int n_q = a.Tq > q_begin ? (int)cdiv(a.Tq - q_begin, BQ) : 0;
+  const int n_steps = n_q * group;
+  f32x16 dk[MT], dv[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) dk[mt] = dv[mt] = zero16();
+  float* dkr = (float*)a.dk + b * a.sdk_b + hk * a.sdk_h + (int64_t)kvw * a.sdk_s;
+  float* dvr = (float*)a.dv + b * a.sdv_b + hk * a.sdv_h + (int64_t)kvw * a.sdv_s;
+  if (n_steps == 0) {  // no query sees these rows
+    if (half == 0 && kvvalid) {
+      f32_store_row<D>(dkr, dk, 1.f, g);
+      f32_store_row<D>(dvr, dv, 1.f, g);
+    }
+    return;
+  }
+
   float4 kf[D / 8], vf[D / 8];
   f32_load_row<D>(kf, (const float*)a.k + b * a.sk_b + hk * a.sk_h + (int64_t)kvw * a.sk_s, kvvalid, g);
   f32_load_row<D>(vf, (const float*)a.v + b * a.sv_b + hk * a.sv_h + (int64_t)kvw * a.sv_s, kvvalid, g);
   F32Offs<D> of;
   of.init();
-  f32x16 dk[MT], dv[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) dk[mt] = dv[mt] = zero16();
-
-  const int q_begin = a.causal ? kv0 : 0;  // top-left causal: rows < kv0 see none
-  const int n_q = a.Tq > q_begin ? (int)cdiv(a.Tq - q_begin, BQ) : 0;
-  const int n_steps = n_q * group;
   F32Dma<D, WAVES> dma;
   dma.init(a.sq_s, a.sdo_s);
   auto issue = [&](int hq, int q0, char* stage) {
@@ -465,7 +474,7 @@ attn_bwd_dkdv_f32(BwdArgs a) {
   };
   // (head, tile) of the current step and of the one being fetched
   int hq = hk * group, qi = 0, hq_n = hq, qi_n = 0;
-  if (n_steps > 0) issue(hq, q_begin, smem);
+  issue(hq, q_begin, smem);
   for (int step = 0; step < n_steps; ++step) {
     wait_vmcnt<0>();
     __syncthreads();
@@ -477,7 +486,7 @@ attn_bwd_dkdv_f32(BwdArgs a) {
     }
     if (step + 1 < n_steps) issue(hq_n, q_begin + BQ * qi_n, smem + ((step + 1) & 1) * STAGE);
     const int qb = q_begin + BQ * qi + 32 * half;  // this wavefront's 32 query rows
-    if (qb >= a.Tq || (a.causal && qb + 31 < kvb)) continue;
+    if (kvb >= a.Tkv || qb >= a.Tq || (a.causal && qb + 31 < kvb)) continue;
     const char* stage = smem + (step & 1) * STAGE;
     const char* Qs = stage + F32Dma<D, WAVES>::template rows_at<SH>(half);
     const char* dOs = Qs + P::BYTES;
@@ -510,8 +519,8 @@ attn_bwd_dkdv_f32(BwdArgs a) {
     return;
   }
   if (half == 0 && kvvalid) {
-    f32_store_row<D>((float*)a.dk + b * a.sdk_b + hk * a.sdk_h + (int64_t)kvw * a.sdk_s, dk, a.scale, g);
-    f32_store_row<D>((float*)a.dv + b * a.sdv_b + hk * a.sdv_h + (int64_t)kvw * a.sdv_s, dv, 1.f, g);
+    f32_store_row<D>(dkr, dk, a.scale, g);
+    f32_store_row<D>(dvr, dv, 1.f, g);
   }
 }
 
@@ -527,8 +536,37 @@ bool f32_share4(int64_t D, bool causal, int64_t blocks) {
   return D == 64 && blocks <= (causal ? 2 : 1) * (int64_t)cu_count();
 }
 
+// Whether the query rows (forward, dQ) stay on the SIMT kernels: a 32 x 32
+// block costs the matrix kernels the same however few of its pairs exist,
+// and a workgroup fills a compute unit (half of one at head_dim 64), while the
+// SIMT kernels take one wavefront a row and one key after the other.  So they
+// win where a row sees at most `few` keys, and where a few rows and keys of
+// very many heads make many workgroups of little work.  Measured, SIMT ->
+// matrix, forward, us:
+//   keys    causal [8, 8] x 64 heads, 64: 7.7 -> 14.2, [13, 13] x 512 11.5 ->
+//     14.3, [14, 14] x 2048, 128: 63 -> 72, against [16, 16] x 64, 128: 12 -> 10
+//   heads, no mask  head_dim 128: 1 x 64 keys x 4096 heads 113 -> 203, x 2048 83 -> 104,
+//     x 1024 85 -> 54; 2 x 128 x 4096 270 -> 338; 4 x 64 x 2048 106 -> 104;
+//     head_dim 64: 1 x 32 x 4096 32 -> 55, 1 x 64 x 4096 59 -> 57, x 2048 53 -> 31
+bool f32_rows_simt(int64_t D, bool causal, int64_t heads, int64_t Tq, int64_t Tkv, int64_t few) {
+  const int64_t keys = causal ? std::min(Tq, Tkv) : Tkv;  // of a row, at most
+  int64_t per = D == 64 ? 64 : heads >= 8 * (int64_t)cu_count() ? 16 : 32;
+  if (keys <= 16) per = D == 64 ? 32 : 16;
+  return keys <= few || Tq * keys <= heads / per;
+}
+constexpr int64_t kF32FewFwd = 13;
+// Backward: keys of a row (dQ), query rows of a head (dK/dV; whatever the
+// group: the matrix kernel takes a step of 64 rows per head).  [16, 16] x 8
+// heads at 128: 24.6 -> 29 us for both, [18, 18] 27 -> 30, [20, 20] x 64 32 -> 30;
+// at 64 [16, 16] 18.5 -> 20, [18, 18] 20 -> 20
+template <int D> constexpr int64_t f32_few_bwd() { return D == 128 ? 18 : 16; }
+
 template <int D>
 int fwd_f32(const FwdArgs& a, hipStream_t st) {
+  if (f32_rows_simt(D, a.causal, (int64_t)a.B * a.H, a.Tq, a.Tkv, kF32FewFwd)) {
+    attn_fwd_simt<float, D / 64><<<(unsigned)((int64_t)a.B * a.H * a.Tq), 64, 0, st>>>(a, D);
+    return check_launch("attention forward (simt)");
+  }
   FwdArgs x = a;
   constexpr int QB = f32_fwd_blocks<D>();
   x.n_tiles = (int)cdiv(a.Tq, 32 * QB);
@@ -550,17 +588,26 @@ int bwd_f32(const BwdArgs& a, hipStream_t st) {
   BwdArgs x = a;
   x.n_tiles = (int)cdiv(a.Tq, 32 * RB);
   const int64_t q_blocks = (int64_t)x.n_tiles * a.B * a.H;
-  const int64_t kv_blocks = cdiv(a.Tkv, 32 * RB) * a.B * a.Hkv;
-  const bool q4 = f32_share4(D, a.causal, q_blocks), kv4 = f32_share4(D, a.causal, kv_blocks);
-  if constexpr (D == 64) {
-    if (q4) attn_bwd_dq_f32<D, 4><<<(unsigned)q_blocks, 256 * RB, 0, st>>>(x);
+  if (f32_rows_simt(D, a.causal, (int64_t)a.B * a.H, a.Tq, a.Tkv, f32_few_bwd<D>())) {
+    const int64_t rows = (int64_t)a.B * a.H * a.Tq;
+    attn_bwd_delta<float><<<(unsigned)cdiv(rows, 4), 256, 0, st>>>(a, D);
+    if (int e = check_launch("attention backward (delta)")) return e;
+    attn_bwd_dq_simt<float, D / 64><<<(unsigned)rows, 64, 0, st>>>(a, D);
+  } else if (f32_share4(D, a.causal, q_blocks)) {
+    if constexpr (D == 64) attn_bwd_dq_f32<D, 4><<<(unsigned)q_blocks, 256 * RB, 0, st>>>(x);
+  } else {
+    attn_bwd_dq_f32<D, 2><<<(unsigned)q_blocks, 128 * RB, 0, st>>>(x);
   }
-  if (!q4) attn_bwd_dq_f32<D, 2><<<(unsigned)q_blocks, 128 * RB, 0, st>>>(x);
   if (int e = check_launch("attention backward (dq, fp32)")) return e;
   x.n_tiles = (int)cdiv(a.Tkv, 32 * RB);
-  if constexpr (D == 64) {
-    if (kv4) attn_bwd_dkdv_f32<D, 4><<<(unsigned)kv_blocks, 256 * RB, 0, st>>>(x);
+  const int64_t kv_blocks = (int64_t)x.n_tiles * a.B * a.Hkv;
+  if (a.Tq <= f32_few_bwd<D>()) {
+    const int64_t kv_rows = (int64_t)a.B * a.Hkv * a.Tkv;
+    attn_bwd_dkdv_simt<float, D / 64><<<(unsigned)kv_rows, 64, 0, st>>>(a, D);
+  } else if (f32_share4(D, a.causal, kv_blocks)) {
+    if constexpr (D == 64) attn_bwd_dkdv_f32<D, 4><<<(unsigned)kv_blocks, 256 * RB, 0, st>>>(x);
+  } else {
+    attn_bwd_dkdv_f32<D, 2><<<(unsigned)kv_blocks, 128 * RB, 0, st>>>(x);
   }
-  if (!kv4) attn_bwd_dkdv_f32<D, 2><<<(unsigned)kv_blocks, 128 * RB, 0, st>>>(x);
   return check_launch("attention backward (dk/dv, fp32)");
 }

@@ -150,11 +150,10 @@ __device__ __forceinline__ void rope_pair(float a, float b, float c, float s, fl
 __host__ __device__ constexpr inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // ---- global -> LDS DMA -----------------------------------------------------
-typedef __attribute__((address_space(3))) void lds_void;
-
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)(uintptr_t)(lds_void*)p;
-}
+// LDS address of a pointer into shared memory: the low half of the generic
+// pointer (the high half is the LDS aperture).  An address space cast would
+// test for null, which the compiler cannot always keep scalar.
+__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)p; }
 
 // One global_load_lds_dwordx4: lane i's 16 bytes at `g` land at LDS byte
 // lds + 16 i (lds must be wave-uniform).  Issued through inline assembly on

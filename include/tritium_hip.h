@@ -166,8 +166,8 @@ int tritium_adamw_step_mixed(const int64_t* table, int n_tensors, int64_t total_
  * lse: [B, H, Tq] float32, natural-log logsumexp of the scaled scores.
  * causal != 0 applies the top-left mask q_pos >= kv_pos; scale = D^-0.5.
  * bf16/fp16 with D in {16, 32, 64, 128, 256} run on MFMA, as does float32
- * with D in {64, 128} and 16-byte aligned rows; anything else on the SIMT
- * path (D <= 1024).  (At D = 256 the backward's dK/dV runs as two
+ * with D in {64, 128} and 16-byte aligned rows that see more than a few
+ * others; anything else on the SIMT path (D <= 1024).  (At D = 256 the backward's dK/dV runs as two
  * launches, dV then dK, each forming S again: the fragments and accumulators
  * of one pass would not fit a wavefront's registers.) */
 int tritium_attention_fwd(const void* q, const void* k, const void* v, void* o, float* lse,

@@ -303,6 +303,20 @@ def test_attention_fp32_matrix_kernels(b, h, hkv, tq, tkv, layout, causal, head_
     _check(torch.float32, b, h, hkv, tq, tkv, head_dim, causal, seed=61, layout=layout)
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_fp32_few_rows(causal, head_dim):
+    # rows that see few others take the SIMT kernels, each of forward, dQ and dK/dV by its
+    # own count: both sides of every line (13 keys forward; 16 or 18 keys or queries
+    # backward; one query of 16 keys in 512 heads), GQA, and keys past the last query's
+    # block (zero gradients, no block computed)
+    for h, hkv, tq, tkv in ((4, 2, 5, 200), (4, 4, 1, 200), (4, 1, 13, 13), (4, 4, 14, 14),
+                            (4, 2, 16, 40), (4, 2, 17, 17), (4, 4, 18, 40), (4, 1, 19, 19),
+                            (4, 2, 300, 13), (4, 4, 300, 17), (2, 2, 300, 19), (2, 2, 40, 300)):
+        _check(torch.float32, 1, h, hkv, tq, tkv, head_dim, causal, seed=76)
+    _check(torch.float32, 64, 8, 8, 1, 16, head_dim, causal, seed=77)
+
+
 @pytest.mark.parametrize("causal", [False, True])
 def test_attention_fp32_large_grid(causal):
     # 640 row tiles: two wavefronts a row block at head_dim 64 (four below 257 or 513)
