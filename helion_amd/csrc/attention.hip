@@ -544,7 +544,7 @@ struct BTile {
 
 // DMA two 64-row tiles (x rows r0.. of x and y, rows clamped to n_rows - 1)
 // into dst and dst + BYTES, spread over the WAVES wavefronts.
-template <typename T, int D, int WAVES>
+template <typename T, int D, int WAVES, bool RAW = false>
 __device__ __forceinline__ void bt_dma2(char* dst, const T* x, int64_t sx, const T* y, int64_t sy,
                                         int r0, int n_rows) {
   typedef BTile<D> P;
@@ -560,7 +560,7 @@ __device__ __forceinline__ void bt_dma2(char* dst, const T* x, int64_t sx, const
     const int row = min(r0 + trow, n_rows - 1);
     const int c = (lane % P::GR) ^ P::key(trow);
     const T* src = (second ? y + (int64_t)row * sy : x + (int64_t)row * sx) + c * 8;
-    dma16(src, __builtin_amdgcn_readfirstlane(lds_addr(dst + (second ? P::BYTES : 0) + part * 1024)));
+    dma16(src, __builtin_amdgcn_readfirstlane(lds_addr<RAW>(dst + (second ? P::BYTES : 0) + part * 1024)));
   }
 }
 
@@ -568,7 +568,7 @@ __device__ __forceinline__ void bt_dma2(char* dst, const T* x, int64_t sx, const
 // row are computed once (init), a full tile then costs one scalar base per
 // tensor and no per-lane address arithmetic; a tile that reaches past
 // n_rows falls back to bt_dma2's clamped rows.
-template <typename T, int D, int WAVES>
+template <typename T, int D, int WAVES, bool RAW = false>
 struct BtDma {
   typedef BTile<D> P;
   static constexpr int PER = 2 * P::DMAS / WAVES;
@@ -597,10 +597,10 @@ struct BtDma {
         const bool second = grp >= P::DMAS;
         dma16s(second ? by : bx, off[i],
                __builtin_amdgcn_readfirstlane(
-                   lds_addr(dst + (second ? P::BYTES : 0) + (grp % P::DMAS) * 1024)));
+                   lds_addr<RAW>(dst + (second ? P::BYTES : 0) + (grp % P::DMAS) * 1024)));
       }
     } else {
-      bt_dma2<T, D, WAVES>(dst, x, sx, y, sy, r0, n_rows);
+      bt_dma2<T, D, WAVES, RAW>(dst, x, sx, y, sy, r0, n_rows);
     }
   }
 };

@@ -146,7 +146,7 @@ __device__ __forceinline__ void f32_store_row(float* p, const f32x16 (&v)[D / 32
 template <int D, int WAVES>
 struct F32Dma {
   typedef BTile<2 * D> P;
-  BtDma<bf16_t, 2 * D, WAVES> dma;
+  BtDma<bf16_t, 2 * D, WAVES, true> dma;
   __device__ __forceinline__ void init(int64_t sx, int64_t sy) { dma.init(2 * sx, 2 * sy); }
   template <int TILES>
   __device__ __forceinline__ void issue(char* dst, const float* x, int64_t sx, const float* y,
@@ -470,7 +470,7 @@ attn_bwd_dkdv_f32(BwdArgs a) {
     if (wave < SH)
       dma4((wave & 1 ? a.delta : a.lse) + row,
            __builtin_amdgcn_readfirstlane(
-               lds_addr(stage + SH * P::BYTES + (wave & 1) * SH * 128 + (wave >> 1) * 256)));
+               lds_addr<true>(stage + SH * P::BYTES + (wave & 1) * SH * 128 + (wave >> 1) * 256)));
   };
   // (head, tile) of the current step and of the one being fetched
   int hq = hk * group, qi = 0, hq_n = hq, qi_n = 0;

@@ -150,10 +150,18 @@ __device__ __forceinline__ void rope_pair(float a, float b, float c, float s, fl
 __host__ __device__ constexpr inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // ---- global -> LDS DMA -----------------------------------------------------
-// LDS address of a pointer into shared memory: the low half of the generic
-// pointer (the high half is the LDS aperture).  An address space cast would
-// test for null, which the compiler cannot always keep scalar.
-__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)p; }
+typedef __attribute__((address_space(3))) void lds_void;
+
+// LDS address of a pointer into shared memory.  RAW: the low half of the
+// generic pointer (the high half is the LDS aperture), without the null test
+// of an address space cast, which the compiler moved to the vector unit in the
+// fp32 attention kernels, with an operand that the assembler rejects.  (The
+// 16-bit forward at head_dim 128 is 7% slower with it at [1, 32, 2048 x 300].)
+template <bool RAW = false>
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  if constexpr (RAW) return (uint32_t)(uintptr_t)p;
+  else return (uint32_t)(uintptr_t)(lds_void*)p;
+}
 
 // One global_load_lds_dwordx4: lane i's 16 bytes at `g` land at LDS byte
 // lds + 16 i (lds must be wave-uniform).  Issued through inline assembly on
