@@ -3249,10 +3249,18 @@ int simt_per_lane(int64_t d) {
 //     16, 2048] 33.2 -> 28.5, no mask [1, 32, 1280] 28.5 -> 24.5, against
 //     [8, 32, 256] 10.2 -> 11.4, [16, 16, 100] 6.2 -> 6.3, no mask [1, 16,
 //     4096] 85 -> 89
-bool split_forward(int64_t D, bool causal, int64_t n_tiles, int64_t blocks) {
+// Fewer keys than queries leave short sweeps, and under the causal mask ever
+// more tiles that see every key and are alike (Tq x Tkv, causal):
+//   head_dim 128  [1, 24, 2048 x 1000] 29.5 -> 35.7, [1, 12, 2048 x 64] 7.0 ->
+//     8.3, [2, 16, 63 x 63] 5.5 -> 5.7, against [1, 12, 2048 x 1000] 24.9 -> 20.2
+//   head_dim 64  [1, 32, 2048 x 500] 16.1 -> 17.5, [1, 12, 2048 x 64] 5.0 ->
+//     5.5, against [1, 32, 2048 x 1000] 24.6 -> 23.2, [1, 8, 2048 x 500] 11.0 -> 8.8
+bool split_forward(int64_t D, bool causal, int64_t n_tiles, int64_t Tkv, int64_t blocks) {
+  const int64_t n = std::min(n_tiles, cdiv(Tkv, kF2BM));  // 128-row steps of the longest sweep
   int half_cus = 1;  // up to so many halves of the compute units in 128-row tiles
-  if (D == 64 && n_tiles > 1) half_cus = causal && n_tiles >= 4 ? 4 : 3;
-  if (D == 128 && causal) half_cus = n_tiles >= 8 ? 3 : n_tiles >= 4 ? 2 : 1;
+  if (D == 64 && n > 1) half_cus = causal && n >= 4 && 2 * n >= n_tiles ? 4 : 3;
+  if (D == 128 && causal) half_cus = n >= 8 && 4 * n >= 3 * n_tiles ? 3 : n >= 4 ? 2 : 1;
+  if (D == 128 && Tkv <= kF2BN) half_cus = 0;  // one K/V tile: half of it empty or soon done
   return D <= 128 && 2 * blocks <= (int64_t)half_cus * cu_count();
 }
 
@@ -3276,7 +3284,7 @@ int fwd_mfma(const FwdArgs& a, int64_t D, hipStream_t st) {
     FwdArgs x = a;
     x.n_tiles = (int)cdiv(a.Tq, kF2BM);
     int64_t blocks = (int64_t)x.n_tiles * a.B * a.H;
-    if (split_forward(D, a.causal, x.n_tiles, blocks)) {
+    if (split_forward(D, a.causal, x.n_tiles, a.Tkv, blocks)) {
       x.n_tiles = (int)cdiv(a.Tq, kF2BM / 2);
       blocks = (int64_t)x.n_tiles * a.B * a.H;
       if (D == 128)
@@ -3326,9 +3334,19 @@ constexpr int kDkvWaves = 4, kDqWaves = 4;
 //     8192] 2163 -> 2374
 //   no mask  [1, 32/8, 1531] 263 -> 210, [1, 16, 1000] 83.6 -> 74.1, against
 //     [4, 32/8, 700] 184 -> 213, [1, 32, 1024] 100 -> 109
-bool split_pairs(bool causal, int64_t n_tiles, int64_t items) {
-  const int half_cus = causal && n_tiles >= 4 ? 2 : 1;  // up to so many halves of the compute units
-  return 2 * items <= (int64_t)half_cus * cu_count();
+// What counts under the mask are the tiles that some query sees, and that
+// their lengths differ (Tq x Tkv, causal; backward alone): [1, 8, 64 x 4096]
+// 20.6 -> 23.6, [1, 8, 256 x 4096] 30.7 -> 32.5, [1, 32, 2048 x 1000] 111 -> 115,
+// against [1, 8, 512 x 4096] 41 -> 37; four and five tiles of items that fill the
+// chip are too short ([1, 60, 512] 44.9 -> 46.7, [1, 48, 512] 43.7 -> 43.3); a
+// single step over a single tile of half the rows gains nothing ([2, 16, 63 x
+// 63] 14.8 -> 15.6).
+bool split_pairs(bool causal, int64_t n_tiles, int64_t Tq, int64_t Tkv, int64_t items) {
+  if (Tq <= 64 && Tkv <= 64) return false;
+  const int64_t n = std::min(n_tiles, cdiv(Tq, kPairBN));
+  int quarter_cus = 2;  // up to so many quarters of the compute units
+  if (causal && n >= 4 && 4 * Tkv >= 3 * Tq) quarter_cus = n >= 6 ? 4 : 3;
+  return 4 * items <= (int64_t)quarter_cus * cu_count();
 }
 
 // The dK/dV pair kernel over the kv tiles of every (batch, kv head): split
@@ -3342,7 +3360,7 @@ int launch_dkdv_pair(const BwdArgs& a, hipStream_t st) {
   const int64_t n_bhk = (int64_t)x.B * x.Hkv;
   const int64_t items = n_bhk * x.n_tiles;
   const int cus = cu_count();
-  if (split_pairs(a.causal, x.n_tiles, items)) {
+  if (split_pairs(a.causal, x.n_tiles, a.Tq, a.Tkv, items)) {
     x.n_tiles = (int)cdiv(a.Tkv, kPairBN / 2);
     attn_bwd_dkdv_pair<T, D, DS, false, 2>
         <<<(unsigned)(n_bhk * x.n_tiles), 64 * kPairWaves, 0, st>>>(x);
@@ -3406,6 +3424,16 @@ bool split_backward(int64_t D, bool causal, int64_t n_tiles, int64_t blocks) {
   return D == 64 && 2 * blocks <= (int64_t)half_cus * cu_count();
 }
 
+// The same for dK/dV with `steps` 64-row tiles of queries to sweep: one or two
+// leave little to halve, and under the mask few kv tiles that see any (Tq x
+// Tkv, causal, backward alone): [1, 16, 64 x 4096] 15.2 -> 17.5, [1, 16, 128 x
+// 4096] 17.5 -> 19.9, [1, 8, 64 x 4096] 11.7 -> 12.4 (no mask 70.2 -> 73.0),
+// against [1, 8, 100 x 4096] 15.6 -> 14.6, [1, 4, 64 x 4096] 10.9 -> 10.7.
+bool split_backward_kv(int64_t D, bool causal, int64_t n_tiles, int64_t steps, int64_t blocks) {
+  const int half_cus = steps > 2 ? 4 : causal && steps == 2 ? 2 : 1;
+  return 2 * blocks <= (int64_t)half_cus * cu_count() && split_backward(D, causal, n_tiles, blocks);
+}
+
 // dQ first: it also computes delta, which the dK/dV kernel reads.
 template <typename T, int D>
 int bwd_v2(const BwdArgs& a, hipStream_t st) {
@@ -3443,7 +3471,7 @@ int bwd_v2(const BwdArgs& a, hipStream_t st) {
   x.n_tiles = (int)cdiv(a.Tkv, 32 * WK);
   int64_t kv_blocks = (int64_t)x.n_tiles * a.B * a.Hkv;
   if constexpr (D == 64) {
-    if (split_backward(D, a.causal, x.n_tiles, kv_blocks)) {
+    if (split_backward_kv(D, a.causal, x.n_tiles, cdiv(a.Tq, 64) * (a.H / a.Hkv), kv_blocks)) {
       x.n_tiles = (int)cdiv(a.Tkv, 16 * WK);
       kv_blocks = (int64_t)x.n_tiles * a.B * a.Hkv;
       attn_bwd_dkdv_v2<T, D, WK, 0, 2><<<(unsigned)kv_blocks, 64 * WK, 0, st>>>(x);

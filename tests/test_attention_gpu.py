@@ -502,6 +502,16 @@ def test_attention_split_pairs(monkeypatch, causal, stored):
                  grads=True)  # 300 whole tiles: neither split nor persistent
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_attention_split_lines_at_unequal_lengths(head_dim):
+    # where few keys meet many queries (or the reverse) under the causal mask the tiles are
+    # alike (or see none), and whole tiles are taken up to smaller grids: shapes on either
+    # side, in the forward, dQ and dK/dV
+    for b, h, tq, tkv in ((1, 24, 1030, 70), (1, 8, 1030, 70), (1, 16, 64, 2100), (1, 4, 100, 2100),
+                          (1, 6, 600, 2100), (1, 12, 1300, 1000), (2, 16, 63, 63), (1, 4, 200, 33)):
+        _check(torch.bfloat16, b, h, h, tq, tkv, head_dim, True, seed=140)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_order_over_uneven_slices(dtype):
     # causal grids whose slices do not divide over the 8 XCDs take their tiles rank by
