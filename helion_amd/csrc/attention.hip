@@ -3798,9 +3798,12 @@ int decode_launch(const void* q, const void* k, const void* v, void* o, float* l
   // wavefronts per (batch, kv head) takes two passes of loads over its keys
   // and writes the result, which costs less than the second launch it saves
   // ([1, 12, 12, 517, 64] 7.3 -> 5.3 us of kernels, 17.0 -> 14.4 us a call;
-  // at twice the bytes, 1000 keys of 128, 11.7 -> 13.3 us).
+  // at twice the bytes, 1000 keys of 128, 11.7 -> 13.3 us), as long as every
+  // compute unit holds one: two heads per kv head, 256 kv heads 12.0 -> 8.5 us
+  // at 270 keys of 128, 15.2 -> 12.9 at 1000 of 64, but 272 kv heads 12.9 ->
+  // 13.7 and 17.4 -> 20.2 (one head: 14.5 -> 12.1 at 512 of 128, 16.4 -> 17.8).
   a.n_splits = dec_splits(B, Hkv, Tkv);
-  const bool single = group <= 2 && a.n_splits > 1 && Tkv * D <= 65536;
+  const bool single = group <= 2 && a.n_splits > 1 && Tkv * D <= 65536 && B * Hkv <= cu_count();
   if (single) a.n_splits = 1;
   const int step = kDecWaves * (64 / (int)(D / 8));
   a.chunk = (int)(cdiv(cdiv(Tkv, a.n_splits), step) * step);

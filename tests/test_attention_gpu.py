@@ -413,6 +413,17 @@ def test_attention_decode_routes(dtype, head_dim, b, h, hkv, kv_len):
     assert_close(lse, e_lse, 1e-4, 1e-4, "lse")
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize(("b", "h", "hkv", "kv_len"), [
+    (128, 4, 2, 300), (129, 4, 2, 300), (257, 1, 1, 511)])
+def test_attention_decode_one_launch_up_to_one_workgroup_a_unit(head_dim, b, h, hkv, kv_len):
+    k, v = (randn((b, hkv, kv_len, head_dim), torch.bfloat16, 80 + i) for i in range(2))
+    q = randn((b, h, 1, head_dim), torch.bfloat16, 82)
+    o = tritium.attention(q, k, v, is_causal=False)
+    eo, _ = oracle.attention.forward(np32(q), np32(k), np32(v), False)
+    assert_close(o, eo, 2e-2, 2e-2, "o")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("e", [12, 20, 30, 36])
