@@ -2785,10 +2785,10 @@ attn_decode_kernel(DecArgs a) {
 // Bound: HBM.  Graph replays, same box, dec_chunk's kernel -> this one, bf16:
 // [8, 32, 8, 8192, 128] 54.0 -> 47.0 us (5.7 TB/s with the combine), [32, 32,
 // 8, 2048, 128] 53.2 -> 47.8, [1, 32, 8, 4096, 128] 18.2 -> 11.6, [10, 12, 3,
-// 9149, 64] 25.1 -> 21.9, [3, 32, 4, 16000, 64] 33.0 -> 17.4, [1, 16, 2,
+// 9149, 64] 23.5 -> 16.6, [3, 32, 4, 16000, 64] 33.0 -> 17.4, [1, 16, 2,
 // 2000, 64] 18.9 -> 7.5; fp16: the first three 57.5 -> 50.6, 56.8 -> 50.2,
-// 17.4 -> 13.4, [10, 12, 3, 9149, 64] 25.4 -> 25.1; with groups of one and two heads it is equal or up
-// to 4% slower, so those stay on the kernel above.
+// 17.4 -> 13.4, [10, 12, 3, 9149, 64] 24.2 -> 19.0; with groups of one and two
+// heads it is equal or up to 4% slower, so those stay on the kernel above.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 template <typename T>
 __device__ __forceinline__ f32x4 mma16(typename Mfma<T>::V a, typename Mfma<T>::V b, f32x4 c) {
@@ -3805,6 +3805,20 @@ int decode_launch(const void* q, const void* k, const void* v, void* o, float* l
   a.n_splits = dec_splits(B, Hkv, Tkv);
   const bool single = group <= 2 && a.n_splits > 1 && Tkv * D <= 65536 && B * Hkv <= cu_count();
   if (single) a.n_splits = 1;
+  // The matrix kernel (groups of three and more heads) holds two workgroups a
+  // compute unit: chunks just past that would run as a second round (fp16
+  // [31, 6, 2, 9304, 64] 41 -> 31 us, bf16 [53, 16, 4, 928, 128] 25.2 -> 22.1).
+  // Where the kv heads alone are more, its long start counts on short caches,
+  // with up to four heads at head_dim 128, vector against matrix kernel: fp16
+  // [128, 32, 8, 16, 128] 9.9 against 11.9 us, 64 keys 12.6 against 15.0, 512
+  // 46 against 44; bf16 16 keys 9.7 against 9.9, 64 equal; fp16 single requests
+  // of up to 12 keys 5.2 against 5.8.
+  const int64_t cus = cu_count();
+  const bool matrix =
+      group > 4 || (group > 2 && (D == 64 || Tkv > (B * Hkv > 2 * cus ? (dtype == kBF16 ? 32 : 256)
+                                                                      : (dtype == kBF16 ? 0 : 12))));
+  if (matrix && a.n_splits > 1 && B * Hkv * a.n_splits > 2 * cus)
+    a.n_splits = (int)std::max<int64_t>(1, 2 * cus / (B * Hkv));
   const int step = kDecWaves * (64 / (int)(D / 8));
   a.chunk = (int)(cdiv(cdiv(Tkv, a.n_splits), step) * step);
   a.sl2 = (float)(1.0 / sqrt((double)D)) * kLog2e;
@@ -3818,8 +3832,9 @@ int decode_launch(const void* q, const void* k, const void* v, void* o, float* l
   attn_decode_kernel<TT, DD, GG, WW><<<(unsigned)blocks, 64 * (WW), 0, st>>>(a)
 #define TRI_DEC_GROUPS(TT, DD)                                      \
   do {                                                              \
-    if (group > 2)                                                  \
+    if (matrix)                                                     \
       attn_decode_mfma<TT, DD><<<(unsigned)blocks, 64 * kDecMWaves, 0, st>>>(a); \
+    else if (group > 2) TRI_DEC_LAUNCH(TT, DD, 4, kDecWaves);       \
     else if (group == 2 && single) TRI_DEC_LAUNCH(TT, DD, 2, 16);   \
     else if (group == 2) TRI_DEC_LAUNCH(TT, DD, 2, kDecWaves);      \
     else if (single) TRI_DEC_LAUNCH(TT, DD, 1, 16);                 \

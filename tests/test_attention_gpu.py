@@ -413,6 +413,21 @@ def test_attention_decode_routes(dtype, head_dim, b, h, hkv, kv_len):
     assert_close(lse, e_lse, 1e-4, 1e-4, "lse")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize(("b", "h", "hkv", "kv_len"), [
+    (65, 24, 8, 32), (65, 32, 8, 33), (65, 24, 8, 256), (65, 32, 8, 257), (2, 12, 4, 12),
+    (2, 16, 4, 13), (33, 12, 4, 600), (33, 24, 4, 600), (257, 6, 2, 300)])
+def test_attention_decode_groups_on_large_and_small_grids(dtype, head_dim, b, h, hkv, kv_len):
+    # groups of 3, 4 and 6: short caches at head_dim 128 on the vector kernel (up to 32 or 256
+    # keys where the kv heads fill the chip, 12 in fp16 else), chunks that fit the chip at once
+    k, v = (randn((b, hkv, kv_len, head_dim), dtype, 80 + i) for i in range(2))
+    q = randn((b, h, 1, head_dim), dtype, 82)
+    o = tritium.attention(q, k, v, is_causal=False)
+    eo, _ = oracle.attention.forward(np32(q), np32(k), np32(v), False)
+    assert_close(o, eo, 2e-2, 2e-2, "o")
+
+
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize(("b", "h", "hkv", "kv_len"), [
     (128, 4, 2, 300), (129, 4, 2, 300), (257, 1, 1, 511)])
