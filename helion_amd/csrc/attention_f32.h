@@ -40,13 +40,16 @@
 //
 // Masked pairs of a partly masked 32 x 32 block are multiplied too, with a
 // weight of zero, and zero times an infinite or NaN element of the other
-// operand is NaN.  So a workgroup with masked pairs whose sums end in any NaN
-// takes its rows again with the SIMT code, which visits the visible pairs
+// operand is NaN.  So where there are masked pairs, rows whose sums end in any
+// NaN are taken again with the SIMT code, which visits the visible pairs
 // only: what a hidden row holds never reaches the result.  The forward does so
 // for an infinite sum too: its weights reach 2^8 (lazy rescaling) where those
 // of the SIMT code reach 1, so values of 1e36 may overflow in its sums alone.
 // (A reference point that follows every row's maximum would do without, and
-// costs the forward another 2%.)
+// costs the forward 2 to 3%.)  It costs the forward under 1% and the backward
+// 1 to 3% ([4, 12, 1024, 64] 235 -> 241 us: other registers in the main loop); a
+// call all of whose rows are NaN takes four times what the SIMT kernels did,
+// one wavefront going through its 32 rows.
 
 // Per-lane byte offsets into a BTile of D fp32 (2 D 16-bit) columns: row
 // granule 2 i + g of row l32 (i < 8; a granule 16 columns of 16 bytes on is
@@ -185,9 +188,10 @@ __device__ __forceinline__ bool f32_any_nan(const f32x16 (&v)[MT]) {
   return nan;
 }
 
-// Whether any lane of the workgroup says so (a scalar).
-__device__ __forceinline__ bool f32_any_lane(bool x) {
-  return __builtin_amdgcn_readfirstlane(__syncthreads_or(x)) != 0;
+// The wavefront's rows (bit l32) of which a lane says so.
+__device__ __forceinline__ uint32_t f32_rows_where(bool x) {
+  const uint64_t m = __builtin_amdgcn_ballot_w64(x);
+  return (uint32_t)m | (uint32_t)(m >> 32);
 }
 
 // Row blocks of 32 per workgroup; SH wavefronts (2 or 4) share each.
@@ -299,12 +303,11 @@ attn_fwd_f32(FwdArgs a) {
         for (int r = 0; r < 16; ++r) o[mt][r] = o[mt][r] * w0 + part[64 * (2 + 16 * mt + r)] * w1;
     }
   }
-  if (f32_any_lane(half == 0 && qvalid && !f32_all_finite(o))) {
-    for (int r = q0 + wave; r < min(q0 + BM, a.Tq); r += WAVES)
-      simt_fwd_row<float, D / 64>(a, D, (int64_t)bh * a.Tq + r);
-    return;
-  }
-  if (half > 0 || !qvalid) return;
+  uint32_t redo = f32_rows_where(half == 0 && qvalid && !f32_all_finite(o));
+  const bool again = (redo >> l32) & 1;
+  for (; redo != 0; redo &= redo - 1)
+    simt_fwd_row<float, D / 64>(a, D, (int64_t)bh * a.Tq + qw0 + __builtin_ctz(redo));
+  if (half > 0 || !qvalid || again) return;
   // no visible key: zeros; visible keys whose scores are all -inf: NaN, as exp(-inf + inf)
   const float inv = l > 0.f ? 1.0f / l : (n_kv > 0 ? __builtin_nanf("") : 0.f);
   f32_store_row<D>((float*)a.o + b * a.so_b + h * a.so_h + (int64_t)qrow * a.so_s, o, inv, g);
@@ -406,13 +409,12 @@ attn_bwd_dq_f32(BwdArgs a) {
     f32_cols<D>(of, Ks, s, dq);
   }
   f32_merge<MT, SH, PART>(reinterpret_cast<float*>(smem) + qb * 64 * 16 * MT + lane, dq, half);
-  if ((a.causal || a.Tkv % 32 != 0) && f32_any_lane(half == 0 && qvalid && f32_any_nan(dq))) {
-    for (int r = q0 + wave; r < min(q0 + BM, a.Tq); r += WAVES)
-      simt_dq_row<float, D / 64>(a, D, (int64_t)bh * a.Tq + r);  // reads the delta stored above
-    return;
-  }
-  if (half == 0 && qvalid)
+  uint32_t redo =
+      a.causal || a.Tkv % 32 != 0 ? f32_rows_where(half == 0 && qvalid && f32_any_nan(dq)) : 0;
+  if (half == 0 && qvalid && !((redo >> l32) & 1))
     f32_store_row<D>((float*)a.dq + b * a.sdq_b + h * a.sdq_h + (int64_t)qrow * a.sdq_s, dq, a.scale, g);
+  for (; redo != 0; redo &= redo - 1)  // reads the delta stored above, before f32_merge's barriers
+    simt_dq_row<float, D / 64>(a, D, (int64_t)bh * a.Tq + qw0 + __builtin_ctz(redo));
 }
 
 // dK and dV: a lane owns one kv row, the query tiles of every head of its
@@ -512,16 +514,15 @@ attn_bwd_dkdv_f32(BwdArgs a) {
   float* part = reinterpret_cast<float*>(smem) + blk * 64 * 16 * MT + lane;
   f32_merge<MT, SH, PART>(part, dk, half);
   f32_merge<MT, SH, PART>(part, dv, half);
-  if ((a.causal || a.Tq % 32 != 0) &&
-      f32_any_lane(half == 0 && kvvalid && (f32_any_nan(dk) || f32_any_nan(dv)))) {
-    for (int r = kv0 + wave; r < min(kv0 + BN, a.Tkv); r += WAVES)
-      simt_dkdv_row<float, D / 64>(a, D, (int64_t)bhk * a.Tkv + r);
-    return;
-  }
-  if (half == 0 && kvvalid) {
+  uint32_t redo = a.causal || a.Tq % 32 != 0
+                      ? f32_rows_where(half == 0 && kvvalid && (f32_any_nan(dk) || f32_any_nan(dv)))
+                      : 0;
+  if (half == 0 && kvvalid && !((redo >> l32) & 1)) {
     f32_store_row<D>(dkr, dk, a.scale, g);
     f32_store_row<D>(dvr, dv, 1.f, g);
   }
+  for (; redo != 0; redo &= redo - 1)
+    simt_dkdv_row<float, D / 64>(a, D, (int64_t)bhk * a.Tkv + kvb + __builtin_ctz(redo));
 }
 
 // Whether four wavefronts share a row block (head_dim 64): `blocks` of 64
