@@ -29,10 +29,13 @@
 // 32 columns of the same row-major tile.  Nothing is transposed and no
 // score leaves the registers.
 //
-// Measured at [4, 12, 1024, 64] causal, forward and backward: 290 us a pass
-// against 9520 us on the SIMT kernels (76 + 107 + 135 us of kernels in the
-// profiler against 2820 + 3374 + 3394), 87 to 99 TFLOP/s each on the blocks
-// they compute; error against float64 6.5e-7 against 8.0e-7.
+// Measured at [4, 12, 1024, 64] causal, forward and backward: 300 us a pass
+// against 9500 us on the SIMT kernels (77 + 111 + 143 us of kernels in the
+// profiler against 2820 + 3374 + 3394), 86 to 93 TFLOP/s each on the blocks
+// they compute; error against float64 6.5e-7 against 8.0e-7.  At head_dim 128,
+// forward / backward alone against SIMT, causal: [4, 12, 1024] 136 / 470 us
+// against 4530 / 8760, [1, 32, 1024] 135 / 292 against 3370 / 6040, [2, 16,
+// 700] 93 / 184 against 1760 / 3090, [8, 12, 128] 25 / 52 against 254 / 470.
 //
 // Numerics: every product, sum and weight is fp32; p = 2^((s * scale - m)
 // log2 e) with the difference formed before the conversion to log2 units, so

@@ -151,10 +151,10 @@ _G_CHUNK_BYTES = 1 << 30
 def _backward_f32(grad_out, h2, w2, target_1d, lse, need_dh, need_dw, ignore_index,
                   chunk_rows: int = 0):
     """fp32 inputs: per vocabulary chunk the HIP kernel recomputes the logits
-    (exact fp32 FMAs) and writes only G = (softmax - onehot) * grad_out /
+    (fp32 products and sums) and writes only G = (softmax - onehot) * grad_out /
     n_valid (``tritium_linear_ce_grad_logits``); dH += G W_c and dW_c = G^T H
     are fp32 library GEMMs on views (cross_entropy.py:928-957 does the same
-    chunking).  A correctness path: the MFMA contractions are 16-bit."""
+    chunking).  The backward's own contractions (``tritium_linear_ce_bwd``) are 16-bit."""
     n_rows, dp = h2.shape
     vocab_size = w2.shape[0]
     dev = h2.device

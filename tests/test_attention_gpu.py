@@ -289,9 +289,11 @@ def test_attention_pingpong_grid():
 
 # fp32 at head_dim 64 and 128 runs the fp32 matrix kernels: 64-row tiles (128
 # query rows a workgroup in the head_dim 128 forward) swept by two wavefronts a
-# row block, or four (head_dim 64, small grids).  Edges: one row, rows and keys just over and under 32, 64 and 128,
-# a half without keys, Tq != Tkv under the top-left mask, GQA, strided module
-# views; the last, rows that are not 16-byte aligned, stays on the SIMT path.
+# row block, or four (head_dim 64, small grids).  Edges: rows and keys just over and
+# under 32, 64 and 128, a half without keys, Tq != Tkv under the top-left mask, GQA,
+# strided module views.  (Rows that see few others -- here a single key, or a single
+# query in dK/dV -- and, further down, rows that are not 16-byte aligned take the SIMT
+# kernels.)
 # Tolerance 1e-5: fp32 sums of at most 300 terms of order 1.
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("causal", [False, True])
@@ -493,7 +495,8 @@ def test_attention_decode_infinite_value():
 @pytest.mark.parametrize("causal", [False, True])
 def test_attention_forward_split_and_whole_tiles(head_dim, causal):
     # small grids take 64-row query tiles whose two wavefronts a row block sweep alternate
-    # 32-key halves (a half without keys, without visible keys, ragged); large ones 128-row tiles
+    # 32-key halves (a half without keys, without visible keys, ragged), at head_dim 128 from
+    # two K/V tiles on; large ones 128-row tiles
     for tq, tkv in ((1, 31), (33, 33), (64, 96), (65, 97), (130, 64), (300, 40), (95, 128)):
         _check(torch.float16, 1, 4, 2, tq, tkv, head_dim, causal, seed=100, grads=False)
     _check(torch.bfloat16, 2, 3, 3, 257, 257, head_dim, causal, seed=101, layout="bthd")
@@ -518,7 +521,7 @@ def test_attention_backward_split_and_whole_tiles(causal):
 def test_attention_split_pairs(monkeypatch, causal, stored):
     # head_dim 128, small grids: 64 kv rows a workgroup, two wavefront pairs a row block on
     # alternate halves of every query tile (a half out of range, masked out, ragged), with
-    # and without the stored dS
+    # and without the stored dS; (33, 33), a single step over one key tile, stays whole
     if not stored:
         monkeypatch.setattr(importlib.import_module("helion_amd.attention"), "DS_WORKSPACE_MAX_BYTES", 0)
     for tq, tkv in ((1, 129), (31, 200), (33, 33), (129, 129), (161, 300), (300, 161), (192, 256)):
