@@ -3834,7 +3834,7 @@ int decode_launch(const void* q, const void* k, const void* v, void* o, float* l
   do {                                                              \
     if (matrix)                                                     \
       attn_decode_mfma<TT, DD><<<(unsigned)blocks, 64 * kDecMWaves, 0, st>>>(a); \
-    else if (group > 2) TRI_DEC_LAUNCH(TT, DD, 4, kDecWaves);       \
+    else if (group > 2) TRI_DEC_LAUNCH(TT, 128, 4, kDecWaves); /* head_dim 128 alone */ \
     else if (group == 2 && single) TRI_DEC_LAUNCH(TT, DD, 2, 16);   \
     else if (group == 2) TRI_DEC_LAUNCH(TT, DD, 2, kDecWaves);      \
     else if (single) TRI_DEC_LAUNCH(TT, DD, 1, 16);                 \
